@@ -67,6 +67,7 @@ struct PrefillParams {
   int64_t kss[4], vss[4];
   int B, Hq, Hkv, D, g, nrep, L;
   float scale_sm;  // log2(e) / sqrt(D)
+  int unit_fast;   // MFMA grid: (units, position blocks) instead of (position blocks, units)
 };
 
 __device__ __forceinline__ f32x4_t mfma_f16(u32x4_t a, u32x4_t b, f32x4_t c) {
@@ -196,14 +197,15 @@ void prefill_mfma_kernel(PrefillParams p) {
   const int j4 = lane >> 4;
   const int c16 = lane & 15;
   const int L = p.L;
-  const int unit = blockIdx.y;  // (batch, KV head)
+  const int unit = p.unit_fast ? blockIdx.x : blockIdx.y;  // (batch, KV head)
   const int b = unit / p.Hkv;
   const int kvh = unit - b * p.Hkv;
 
   // rows (position block, head of the group), position-block major; heavy blocks launch first
+  // (launch_mfma)
   const int npb = (L + QW - 1) / QW;
   const int rows = npb * p.nrep;
-  const int wg = (int)gridDim.x - 1 - (int)blockIdx.x;
+  const int wg = p.unit_fast ? (int)(gridDim.y - 1 - blockIdx.y) : (int)(gridDim.x - 1 - blockIdx.x);
   const int row = wg * NW + wave;
   const bool active = row < rows;
   const int pb = active ? row / p.nrep : 0;
@@ -574,12 +576,20 @@ bool prefill_mfma_ok(const PrefillParams& p) {
   return true;
 }
 
+// Workgroup order: the units vary fastest, so the heaviest position block of every (batch, KV head)
+// launches first and the lightest blocks fill the end, and with 8 units each XCD keeps one head's
+// K and V in its L2. With the position blocks fastest, the last unit's heaviest blocks started
+// when the others were done: batch 1, 8 KV heads, L = 4096 442 -> 296 us, 8192 1278 -> 1060 us,
+// 16384 4143 -> 3970 us; batch 2, L = 777 63.7 -> 56.0 us. (More than 65535 position blocks do not
+// fit grid.y and keep the position blocks in grid.x.)
 template <int G>
-void launch_mfma(const PrefillParams& p, hipStream_t st) {
+void launch_mfma(PrefillParams p, hipStream_t st) {
   const int64_t npb = ((int64_t)p.L + QW - 1) / QW;
   const int64_t nwg = (npb * p.nrep + NW - 1) / NW;
-  hipLaunchKernelGGL((prefill_mfma_kernel<G>), dim3((unsigned)nwg, (unsigned)(p.B * p.Hkv)),
-                     dim3(256), 0, st, p);
+  const unsigned units = (unsigned)(p.B * p.Hkv);
+  p.unit_fast = nwg <= 65535;
+  const dim3 grid = p.unit_fast ? dim3(units, (unsigned)nwg) : dim3((unsigned)nwg, units);
+  hipLaunchKernelGGL((prefill_mfma_kernel<G>), grid, dim3(256), 0, st, p);
 }
 
 }  // namespace
