@@ -4,6 +4,12 @@ Only plain pointers, sizes and strides cross the boundary: each torch tensor is 
 LQTensor (data pointer, dtype code, rank, shape, strides in elements). Every compute entry point
 launches on the caller's current HIP stream and never synchronizes. There is no CPU fallback:
 the library must be built (python -m layer_quant_amd.build) and tensors must live on a GPU.
+
+The per-step calls go through the host binding (csrc/host_binding.cpp) when their arguments are
+plain: it fills the descriptors natively and calls the same entry points, about 1 us where building
+them through ctypes takes 2 us per tensor. It declines everything else (a tensor off the GPU or on
+another device, a subclass, an unknown dtype, rank above 4), and the ctypes path below then raises
+or runs the call.
 """
 from __future__ import annotations
 
@@ -93,6 +99,7 @@ class LQError(RuntimeError):
 
 _P = ctypes.POINTER(LQTensor)
 _lib = None
+_host = None  # the bound host binding, or False when it is not built
 _lib_lock = threading.Lock()
 
 
@@ -158,6 +165,34 @@ def lib() -> ctypes.CDLL:
                 _declare(handle)
                 _lib = handle
     return _lib
+
+
+# entry points that the host binding calls, in the order of its bind()
+_HOST_ENTRIES = (
+    "lq_int4_pack_kv", "lq_int4_pack_kv_pair", "lq_int4_decode_attention_workspace",
+    "lq_int4_decode_attention", "lq_int4_decode_attention_pack", "lq_int4_prefill_attention",
+    "lq_mx_encode", "lq_mx_state_update", "lq_mx_state_update_device_step",
+    "lq_selective_state_update",
+)
+
+
+def host_binding():
+    """The host binding bound to the loaded library, or False when it is not built."""
+    global _host
+    if _host is None:
+        handle = lib()
+        with _lib_lock:
+            if _host is None:
+                try:
+                    from . import _lq_host
+                except ImportError:
+                    _host = False
+                else:
+                    _lq_host.bind(torch._C._cuda_getCurrentRawStream, *(
+                        ctypes.cast(getattr(handle, name), ctypes.c_void_p).value
+                        for name in _HOST_ENTRIES))
+                    _host = _lq_host
+    return _host
 
 
 def last_error() -> str:
@@ -248,6 +283,11 @@ def diagnostic(*names: str, on: bool = True):
 def int4_pack_kv(x: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor,
                  positions: torch.Tensor, group_size: int) -> None:
     """Quantize x [B, Hkv, T, D] into rows `positions` of the packed cache (in place)."""
+    host = _host or host_binding()
+    if host:
+        rc = host.int4_pack_kv(x, packed, scale, positions, group_size)
+        if rc is not None:
+            return check(rc, "lq_int4_pack_kv")
     dev = _require_gpu(x, packed, scale, positions)
     rc = lib().lq_int4_pack_kv(desc(x), desc(packed), desc(scale), desc(positions),
                                int(group_size), _stream(dev))
@@ -258,6 +298,12 @@ def int4_pack_kv_pair(k: torch.Tensor, v: torch.Tensor, k_packed: torch.Tensor,
                       v_packed: torch.Tensor, k_scale: torch.Tensor, v_scale: torch.Tensor,
                       positions: torch.Tensor, group_size: int) -> None:
     """int4_pack_kv of a layer's K and V in one launch."""
+    host = _host or host_binding()
+    if host:
+        rc = host.int4_pack_kv_pair(k, v, k_packed, v_packed, k_scale, v_scale, positions,
+                                    group_size)
+        if rc is not None:
+            return check(rc, "lq_int4_pack_kv_pair")
     dev = _require_gpu(k, v, k_packed, v_packed, k_scale, v_scale, positions)
     rc = lib().lq_int4_pack_kv_pair(desc(k), desc(v), desc(k_packed), desc(v_packed),
                                     desc(k_scale), desc(v_scale), desc(positions),
@@ -277,11 +323,16 @@ class _Workspace:
     def get(self, device: torch.device, stream: int, nbytes: int) -> torch.Tensor | None:
         if nbytes == 0:
             return None
-        key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
+        index = device.index if device.index is not None else torch.cuda.current_device()
+        return self.on_index(index, stream, nbytes)
+
+    def on_index(self, index: int, stream: int, nbytes: int) -> torch.Tensor:
+        key = (index, stream)
         with self._lock:
             buf = self._bufs.get(key)
             if buf is None or buf.numel() < nbytes:
-                buf = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+                buf = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8,
+                                  device=torch.device("cuda", index))
                 self._bufs[key] = buf
             return buf
 
@@ -300,6 +351,14 @@ def int4_decode_attention(q: torch.Tensor, k_packed: torch.Tensor, v_packed: tor
                           mask: torch.Tensor | None, out: torch.Tensor, seq_len: int,
                           num_key_value_groups: int, group_size: int) -> torch.Tensor:
     """q_len=1 attention of q [B, Hq, 1, D] (or [B, Hq, D]) over the packed cache -> out."""
+    host = _host or host_binding()
+    if host:
+        rc = host.int4_decode_attention(q, k_packed, v_packed, k_scale, v_scale, mask, out,
+                                        seq_len, num_key_value_groups, group_size,
+                                        _workspace.on_index)
+        if rc is not None:
+            check(rc, "lq_int4_decode_attention")
+            return out
     dev = _require_gpu(q, k_packed, v_packed, k_scale, v_scale, mask, out)
     stream = _stream(dev)
     need = int4_decode_attention_workspace(q.shape[0], q.shape[1], k_packed.shape[1],
@@ -321,6 +380,14 @@ def int4_decode_attention_pack(q: torch.Tensor, k_new: torch.Tensor, v_new: torc
     """int4_pack_kv_pair of the new token k_new, v_new [B, Hkv, 1, D] into cache row
     seq_len - 1, then int4_decode_attention over keys [0, seq_len) -> out; one launch on the MFMA
     path."""
+    host = _host or host_binding()
+    if host:
+        rc = host.int4_decode_attention_pack(q, k_new, v_new, k_packed, v_packed, k_scale, v_scale,
+                                             mask, out, seq_len, num_key_value_groups, group_size,
+                                             _workspace.on_index)
+        if rc is not None:
+            check(rc, "lq_int4_decode_attention_pack")
+            return out
     dev = _require_gpu(q, k_new, v_new, k_packed, v_packed, k_scale, v_scale, mask, out)
     stream = _stream(dev)
     need = int4_decode_attention_workspace(q.shape[0], q.shape[1], k_packed.shape[1],
@@ -355,6 +422,13 @@ def int4_prefill_attention(q: torch.Tensor, k_packed: torch.Tensor, v_packed: to
                            k_scale: torch.Tensor, v_scale: torch.Tensor, out: torch.Tensor,
                            num_key_value_groups: int, group_size: int) -> torch.Tensor:
     """Causal attention of q [B, Hq, L, D] over cache keys 0 .. t for position t -> out."""
+    host = _host or host_binding()
+    if host:
+        rc = host.int4_prefill_attention(q, k_packed, v_packed, k_scale, v_scale, out,
+                                         num_key_value_groups, group_size)
+        if rc is not None:
+            check(rc, "lq_int4_prefill_attention")
+            return out
     dev = _require_gpu(q, k_packed, v_packed, k_scale, v_scale, out)
     rc = lib().lq_int4_prefill_attention(desc(q), desc(k_packed), desc(v_packed), desc(k_scale),
                                          desc(v_scale), desc(out), int(num_key_value_groups),
@@ -367,6 +441,12 @@ def mx_encode(state: torch.Tensor, q_state: torch.Tensor, shared_exp: torch.Tens
               micro_exp: torch.Tensor, format_bits: int,
               round_mode: int = ROUND_NEAREST_EVEN, uniform: torch.Tensor | None = None,
               seed: int = 0, rng_offset: int = 0) -> None:
+    host = _host or host_binding()
+    if host:
+        rc = host.mx_encode(state, q_state, shared_exp, micro_exp, uniform, format_bits, round_mode,
+                            seed, rng_offset)
+        if rc is not None:
+            return check(rc, "lq_mx_encode")
     dev = _require_gpu(state, q_state, shared_exp, micro_exp, uniform)
     rc = lib().lq_mx_encode(desc(state), desc(q_state), desc(shared_exp), desc(micro_exp),
                             int(format_bits), int(round_mode), desc(uniform),
@@ -390,6 +470,14 @@ def mx_state_update(q_state, shared_exp, micro_exp, x, dt, dt_bias, A, B, C, D, 
     """The fused MX update in place. With `step` (an int64 [1] tensor on the device) the counter
     offset is rng_offset + step * B*H*P*N, read by the kernel (lq_mx_state_update_device_step):
     graph-capturable, with the caller advancing `step`."""
+    host = _host or host_binding()
+    if host:
+        rc = host.mx_state_update(q_state, shared_exp, micro_exp, x, dt, dt_bias, A, B, C, D, z, out,
+                                  uniform, step, format_bits, dt_softplus, round_mode, seed,
+                                  rng_offset)
+        if rc is not None:
+            check(rc, "lq_mx_state_update" if step is None else "lq_mx_state_update_device_step")
+            return out
     dev = _require_gpu(q_state, shared_exp, micro_exp, x, dt, dt_bias, A, B, C, D, z, out,
                        uniform, step)
     args = (desc(q_state), desc(shared_exp), desc(micro_exp), desc(x), desc(dt), desc(dt_bias),
@@ -409,6 +497,12 @@ def mx_state_update(q_state, shared_exp, micro_exp, x, dt, dt_bias, A, B, C, D, 
 
 def selective_state_update(state, x, dt, dt_bias, A, B, C, D, z, out,
                            dt_softplus: bool) -> torch.Tensor:
+    host = _host or host_binding()
+    if host:
+        rc = host.selective_state_update(state, x, dt, dt_bias, A, B, C, D, z, out, dt_softplus)
+        if rc is not None:
+            check(rc, "lq_selective_state_update")
+            return out
     dev = _require_gpu(state, x, dt, dt_bias, A, B, C, D, z, out)
     rc = lib().lq_selective_state_update(
         desc(state), desc(x), desc(dt), desc(dt_bias), desc(A), desc(B), desc(C), desc(D),
