@@ -8,8 +8,8 @@
 // per group) covers group sizes whose g/2 is not a power of two up to 64. int4_pack_rows_kernel
 // takes the common layout (contiguous rows, 16-byte aligned, g a multiple of 8): one lane per 8
 // values of each of 4 rows (16- or 32-byte loads issued together, 4-byte stores), g/8 lanes per
-// group, and the division by the scale done as a product with the reciprocal wherever that
-// provably gives the same level.
+// group, and the division by the scale done as a corrected product with its reciprocal, which gives
+// the same levels (pack_levels).
 // All kernels take up to two tensors (blockIdx.y picks one): lq_int4_pack_kv_pair packs a layer's
 // K and V in one launch.
 #include <algorithm>
@@ -107,41 +107,73 @@ __device__ __forceinline__ void decode8(const Raw8<DT>& r, float (&v)[8]) {
   }
 }
 
+// max(|a|, |b|, c), NaN if any of them is NaN (c >= 0): one v_maximum3_f32
+__device__ __forceinline__ float abs_maximum3(float a, float b, float c) {
+  float r;
+  asm("v_maximum3_f32 %0, |%1|, |%2|, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
+// The largest |v| of NV values with NaNs ignored; `odd` when one of them is NaN or infinite (the
+// values then take pack_levels' division).
+template <int NV>
+__device__ __forceinline__ float group_absmax(const float (&v)[NV], bool& odd) {
+  float amax = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NV; i += 2) amax = abs_maximum3(v[i], v[i + 1], amax);
+  odd = !(amax < INFINITY);
+  if (odd) {  // rare
+    amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) amax = fmaxf(amax, fabsf(v[i]));
+  }
+  return amax;
+}
+
 // The packed nibbles of NV values of one group (NV / 8 words, two's-complement levels, the even
 // value in the low nibble), equal to clamp(rint(RN(x / scale)), -8, 7) of the IEEE quotient bit
-// for bit. With y = RN(x * rcp(scale)) (v_rcp_f32 within 1 ulp), |y - RN(x / scale)| <=
-// |x / scale| * (2^-23 + 2^-23 + 2^-24) <= 2^-19 for |x / scale| <= 8, so when y lies more than
-// 2^-17 from every half-integer both round to the same integer (no half-integer lies between
-// them); a lane with a value closer than that (or a non-finite one, or a non-finite scale)
-// recomputes its levels with the IEEE division. t = RN(y + 1.5 * 2^23) is y rounded to an integer
-// k (ties to even) held in the low mantissa bits as k + 2^22, so its low 4 bits are k's
-// two's-complement nibble; |k| <= 7 here because |x| <= absmax and scale >= absmax / 7 rounded.
+// for bit. With y = RN(1 / scale) (one IEEE division per group), q0 = RN(x y), r = x - q0 scale (a
+// fused multiply-add, exact) and q = RN(q0 + r y), q is the IEEE quotient or, for rare pairs, its
+// neighbour; rint(q) = rint(RN(x / scale)) for every pair of fp32 x and scale (checked on the CPU
+// for every fp32 mantissa of x against the scales that put the quotient next to each half-integer,
+// tests/native/pack_levels.c). k = rint(q) comes from adding and subtracting 1.5 * 2^23. |k| <= 7,
+// because |x| <= absmax and scale >= absmax / 7 rounded. `odd` groups (a NaN or infinite value, or
+// scale) divide: NaN and x / inf give level 0.
+// Ties are common, not rare: in bf16 a value is exactly half its group's absmax, i.e. 3.5 scales,
+// in about one group of 15, so a product with v_rcp_f32 that sent lanes near a half-integer to the
+// division sent nearly every wave there (about 27 instructions per value; here about 8). K and V of
+// 16384 tokens, 8 heads, in the kernel trace: g = 32 26.3 -> 14.6 us (88 MB, 6.0 TB/s), g = 64
+// 28.5 -> 16.3, g = 128 (the row kernel) 30.4 -> 21.5 us.
+// The levels join as numbers: four give sum (k_i + 8) 16^i in [0, 65535], exact in fp32, in the low
+// 16 bits of that sum + 2^23 (three fmas and an add); the xor with 8 per nibble makes them two's
+// complement.
 template <int NV>
-__device__ __forceinline__ void pack_levels(const float (&v)[NV], float scale,
+__device__ __forceinline__ void pack_levels(const float (&v)[NV], float scale, bool odd,
                                             uint32_t (&words)[NV / 8]) {
   constexpr float C = 12582912.0f;  // 1.5 * 2^23
-  const float rcp = __builtin_amdgcn_rcpf(scale);
-  float t[NV];
-  bool exact = !(scale < INFINITY);
+  const float y = 1.0f / scale;
+  float k[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const float y = v[i] * rcp;
-    t[i] = y + C;
-    exact |= !(fabsf(y - (t[i] - C)) < 0.5f - 0x1p-17f);
+    const float q0 = v[i] * y;
+    const float q = __builtin_fmaf(__builtin_fmaf(-q0, scale, v[i]), y, q0);
+    k[i] = (q + C) - C;
   }
-  if (exact) {  // rare
+  if (odd || !(scale < INFINITY)) {  // rare
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int q = min(max((int)rintf(v[i] / scale), -8), 7);
-      t[i] = (float)q + C;
-    }
+    for (int i = 0; i < NV; ++i) k[i] = (float)min(max((int)rintf(v[i] / scale), -8), 7);
   }
 #pragma unroll
   for (int w = 0; w < NV / 8; ++w) {
-    uint32_t word = 0;
+    uint32_t half[2];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) word |= (__float_as_uint(t[8 * w + i]) & 15u) << (4 * i);
-    words[w] = word;
+    for (int h = 0; h < 2; ++h) {
+      const float* q = &k[8 * w + 4 * h];
+      const float sum = __builtin_fmaf(__builtin_fmaf(q[3], 16.0f, q[2]), 256.0f,
+                                       __builtin_fmaf(q[1], 16.0f, q[0]));
+      half[h] = __float_as_uint(sum + (8388608.0f + 34952.0f));  // 8 (1 + 16 + 256 + 4096) = 34952
+    }
+    words[w] = __builtin_amdgcn_perm(half[1], half[0], 0x05040100u) ^ 0x88888888u;
   }
 }
 
@@ -149,14 +181,13 @@ __device__ __forceinline__ void pack_levels(const float (&v)[NV], float scale,
 // active), and the group's scale (levels as in pack_levels).
 template <int L8>
 __device__ __forceinline__ uint32_t quantize8(const float (&v)[8], float& scale) {
-  float amax = 0.0f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
+  bool odd;
+  float amax = group_absmax<8>(v, odd);
 #pragma unroll
   for (int o = L8 >> 1; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
   scale = fmaxf(amax / 7.0f, 1.0e-8f);
   uint32_t word[1];
-  pack_levels<8>(v, scale, word);
+  pack_levels<8>(v, scale, odd, word);
   return word[0];
 }
 
@@ -179,6 +210,8 @@ __global__ __launch_bounds__(256) void int4_pack_groups_kernel(PackPair pair, in
   const int h = (int)blockIdx.y - b * p.H;
   const int64_t xe = b * p.x.s[0] + h * p.x.s[1] + t * p.x.s[2] + G * k;
   constexpr int NL = G / 8;
+  // the token's row goes out with the values (loaded before the stores, it was one more round trip)
+  const int64_t pos = p.positions != nullptr ? p.positions[t * p.pos_stride] : p.fixed_pos + t;
   Raw8<DT> raw[NL];
 #pragma unroll
   for (int i = 0; i < NL; ++i) raw[i] = load8<DT>(p.x.data, xe + 8 * i);
@@ -190,15 +223,11 @@ __global__ __launch_bounds__(256) void int4_pack_groups_kernel(PackPair pair, in
 #pragma unroll
     for (int u = 0; u < 8; ++u) v[8 * i + u] = w[u];
   }
-  float amax = 0.0f;
-#pragma unroll
-  for (int i = 0; i < G; ++i) amax = fmaxf(amax, fabsf(v[i]));
-  const float scale = fmaxf(amax / 7.0f, 1.0e-8f);
+  bool odd;
+  const float scale = fmaxf(group_absmax<G>(v, odd) / 7.0f, 1.0e-8f);
   uint32_t words[G / 8];
-  pack_levels<G>(v, scale, words);
-  if (gid >= total) return;
-  const int64_t pos = p.positions != nullptr ? p.positions[t * p.pos_stride] : p.fixed_pos + t;
-  if (pos < 0 || pos >= p.cap) return;
+  pack_levels<G>(v, scale, odd, words);
+  if (gid >= total || pos < 0 || pos >= p.cap) return;
   uint8_t* dst = p.packed + b * p.ps[0] + h * p.ps[1] + pos * p.ps[2] + (G / 2) * k;
   if constexpr (G == 16) {
     *(uint2*)dst = make_uint2(words[0], words[1]);

@@ -1,0 +1,42 @@
+"""The prompt pack kernels' level arithmetic on the GPU: the same bytes and scales as the decode
+token's kernel, which divides every value by its scale, on ties, extremes, NaN and infinities."""
+import pytest
+import torch
+
+from layer_quant_amd import _abi
+
+pytestmark = pytest.mark.gpu
+
+
+def _values(t, d, dtype, gen):
+    x = torch.randn(t, d, generator=gen)
+    x[0::8] = torch.randint(-14, 15, (len(x[0::8]), d), generator=gen) / 4.0  # ties: 14 quarters = 7 halves
+    x[1::8, 3] = 2 * x[1::8, 4]                   # a value that may be half the absmax
+    x[2::8] *= 1e-9                               # the 1e-8 scale floor
+    x[3::8] *= 3e4
+    x[4, 5], x[4, 37], x[12, 70] = float("nan"), float("inf"), float("-inf")
+    x[20] = float("nan")
+    x[28] = 0.0
+    if dtype == torch.float32:
+        x[36] *= 1e38
+        x[44] *= 1e-39
+    return x.to(dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("g", [8, 16, 32, 64, 128])
+def test_prompt_levels_equal_token_levels(gpu, dtype, g):
+    b, h, t, d = 1, 2, 333, 128
+    gen = torch.Generator().manual_seed(g)
+    x = torch.stack([_values(t, d, dtype, gen) for _ in range(b * h)]).view(b, h, t, d).to(gpu)
+
+    def cache():
+        return (torch.zeros(b, h, t, d // 2, dtype=torch.uint8, device=gpu),
+                torch.zeros(b, h, t, d // g, device=gpu))
+
+    prompt, token = cache(), cache()
+    _abi.int4_pack_kv(x, *prompt, torch.arange(t, device=gpu), g)
+    for i in range(t):  # one token per call: the one-lane-per-byte kernel
+        _abi.int4_pack_kv(x[:, :, i:i + 1], *token, torch.tensor([i], device=gpu), g)
+    assert torch.equal(prompt[0], token[0])
+    assert torch.equal(prompt[1], token[1])
