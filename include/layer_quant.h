@@ -159,6 +159,24 @@ int lq_int4_pack_kv_pair(const lq_tensor* k, const lq_tensor* v, const lq_tensor
                          void* stream);
 
 /*
+ * Largest of positions [n] i64 (n >= 1, any stride), written to *host_slot, 8 bytes of pinned host
+ * memory (hipHostMalloc), when the stream reaches the call; the caller waits for that with an event
+ * or the stream. One workgroup: meant for the few thousand positions of a prompt.
+ * Replaces positions.max().item() of the reference's cache update (hybrid_quant/
+ * int4_8b_attention.py:515, 666): a reduction, a copy, and a wait for all the stream's work.
+ */
+int lq_max_position(const lq_tensor* positions, void* host_slot, void* stream);
+
+/*
+ * Additive key bias of a 2-D keep-mask: bias[b, 0, 0, n] = keep[b, n] != 0 ? 0 : -inf.
+ *   keep [B, S] u8/i8/i32/i64/f16/bf16/f32, any strides (a bool tensor's bytes as u8);
+ *   bias [B, 1, 1, S] f32
+ * Replaces the torch expression of the reference (hybrid_quant/int4_8b_attention.py:582-588) by one
+ * launch.
+ */
+int lq_keep_mask_bias(const lq_tensor* keep, const lq_tensor* bias, void* stream);
+
+/*
  * Workspace bytes that lq_int4_decode_attention needs for this shape (0 if none).
  * No counterpart in the reference (its decode kernel has no split-K); it sizes the split-K
  * partials of the kernel below. A workspace (256-byte aligned) starts with

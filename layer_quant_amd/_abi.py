@@ -76,6 +76,8 @@ EXPORTED_SYMBOLS = (
     "lq_mx_state_update",
     "lq_mx_state_update_device_step",
     "lq_selective_state_update",
+    "lq_max_position",
+    "lq_keep_mask_bias",
 )
 
 
@@ -147,6 +149,10 @@ def _declare(lib: ctypes.CDLL) -> None:
         ctypes.c_void_p]
     lib.lq_selective_state_update.restype = ctypes.c_int
     lib.lq_selective_state_update.argtypes = [_P] * 10 + [ctypes.c_int, ctypes.c_void_p]
+    lib.lq_max_position.restype = ctypes.c_int
+    lib.lq_max_position.argtypes = [_P, ctypes.c_void_p, ctypes.c_void_p]
+    lib.lq_keep_mask_bias.restype = ctypes.c_int
+    lib.lq_keep_mask_bias.argtypes = [_P, _P, ctypes.c_void_p]
 
 
 def lib() -> ctypes.CDLL:
@@ -172,7 +178,7 @@ _HOST_ENTRIES = (
     "lq_int4_pack_kv", "lq_int4_pack_kv_pair", "lq_int4_decode_attention_workspace",
     "lq_int4_decode_attention", "lq_int4_decode_attention_pack", "lq_int4_prefill_attention",
     "lq_mx_encode", "lq_mx_state_update", "lq_mx_state_update_device_step",
-    "lq_selective_state_update",
+    "lq_selective_state_update", "lq_max_position", "lq_keep_mask_bias",
 )
 
 
@@ -309,6 +315,78 @@ def int4_pack_kv_pair(k: torch.Tensor, v: torch.Tensor, k_packed: torch.Tensor,
                                     desc(k_scale), desc(v_scale), desc(positions),
                                     int(group_size), _stream(dev))
     check(rc, "lq_int4_pack_kv_pair")
+
+
+class _PendingMax:
+    """One thread's pinned slot and event on one device. wait() ends the use that start() began;
+    the owner calls it before start() is called again, also when the work in between raises."""
+
+    def __init__(self):
+        self._pinned = torch.zeros(1, dtype=torch.int64, pin_memory=True)
+        self.address = self._pinned.data_ptr()
+        self._value = ctypes.c_int64.from_address(self.address)
+        self._event = torch.cuda.Event()
+
+    def record(self, device: int) -> None:
+        self._event.record(torch.cuda.current_stream(device))
+
+    def wait(self) -> int:
+        self._event.synchronize()
+        return self._value.value
+
+
+class _PendingMaxima(threading.local):
+    def __init__(self):
+        self.by_device: dict[int, _PendingMax] = {}
+
+
+_pending_maxima = _PendingMaxima()
+# above this, torch's reduction over many workgroups is the faster one
+MAX_POSITIONS = 1 << 16
+
+
+def start_max_position(positions) -> _PendingMax | None:
+    """Starts reading the largest of `positions` back to the host, behind the work that is on the
+    current stream now; .wait() gives it without waiting for work launched since. None when positions
+    is not a plain 1-D int64 tensor on a GPU, or the stream is being captured: the caller then
+    uses positions.max().item()."""
+    if type(positions) is not torch.Tensor or positions.dtype != torch.int64 \
+            or positions.dim() != 1 or not positions.is_cuda \
+            or not 1 <= positions.numel() <= MAX_POSITIONS:
+        return None
+    host = _host or host_binding()
+    if not host or torch.cuda.is_current_stream_capturing():
+        return None
+    device = positions.get_device()
+    pending = _pending_maxima.by_device.get(device)
+    if pending is None:
+        pending = _pending_maxima.by_device[device] = _PendingMax()
+    rc = host.max_position(positions, pending.address)
+    if rc is None:
+        return None
+    check(rc, "lq_max_position")
+    pending.record(device)
+    return pending
+
+
+def keep_mask_bias(keep: torch.Tensor, batch: int, seq_len: int,
+                   device: torch.device) -> torch.Tensor | None:
+    """The additive fp32 bias [batch, 1, 1, seq_len] of a keep-mask [batch, seq_len] (0 where it is
+    not zero, -inf elsewhere) in one launch; None when the mask is not a plain tensor of that shape
+    on `device` with an ABI dtype (or bool)."""
+    if type(keep) is not torch.Tensor or keep.device != device or keep.shape != (batch, seq_len):
+        return None
+    host = _host or host_binding()
+    if not host:
+        return None
+    if keep.dtype == torch.bool:
+        keep = keep.view(torch.uint8)
+    bias = torch.empty((batch, 1, 1, seq_len), device=device, dtype=torch.float32)
+    rc = host.keep_mask_bias(keep, bias)
+    if rc is None:
+        return None
+    check(rc, "lq_keep_mask_bias")
+    return bias
 
 
 class _Workspace:

@@ -27,6 +27,8 @@ struct Entries {
   decltype(&lq_mx_state_update) update;
   decltype(&lq_mx_state_update_device_step) update_step;
   decltype(&lq_selective_state_update) ssm;
+  decltype(&lq_max_position) max_position;
+  decltype(&lq_keep_mask_bias) keep_mask;
 } entries;
 constexpr int kEntries = sizeof(Entries) / sizeof(void*);
 
@@ -277,6 +279,23 @@ PyObject* py_ssm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// positions, address of the pinned host slot
+PyObject* py_max_position(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (!has_args(n, 2)) return nullptr;
+  Tensors<1> t;
+  int64_t slot;
+  LQ_NOT_PLAIN(!t.add_all(a) || !to_int64(a[1], slot));
+  return launch(t.device, [&](void* s) { return entries.max_position(t.ptr[0], (void*)slot, s); });
+}
+
+// keep-mask, bias
+PyObject* py_keep_mask(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (!has_args(n, 2)) return nullptr;
+  Tensors<2> t;
+  LQ_NOT_PLAIN(!t.add_all(a));
+  return launch(t.device, [&](void* s) { return entries.keep_mask(t.ptr[0], t.ptr[1], s); });
+}
+
 // bind(current raw stream function, addresses of the entry points in the order of Entries)
 PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!has_args(n, 1 + kEntries)) return nullptr;
@@ -320,6 +339,8 @@ PyMethodDef methods[] = {LQ_METHOD("bind", py_bind),
                          LQ_METHOD("mx_encode", py_encode),
                          LQ_METHOD("mx_state_update", py_update),
                          LQ_METHOD("selective_state_update", py_ssm),
+                         LQ_METHOD("max_position", py_max_position),
+                         LQ_METHOD("keep_mask_bias", py_keep_mask),
                          {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_lq_host", nullptr, -1, methods,

@@ -120,9 +120,16 @@ def _pack_kv_into_cache(cache: Int4KVLayerCache, key_states: torch.Tensor,
                         group_size: int) -> None:
     """INT4-pack K and V [B, Hkv, q_len, D] into rows `positions` (ia.py:477-515); one launch
     for both (the reference launches _pack_int4_kv_kernel once for K and once for V)."""
-    _abi.int4_pack_kv_pair(key_states, value_states, cache.k_packed, cache.v_packed,
-                           cache.k_scale, cache.v_scale, positions, group_size)
-    cache.length = max(cache.length, int(positions.max().item()) + 1)
+    # the length's read-back goes out before the pack, so that the host does not wait for the pack
+    pending = _abi.start_max_position(positions)
+    try:
+        _abi.int4_pack_kv_pair(key_states, value_states, cache.k_packed, cache.v_packed,
+                               cache.k_scale, cache.v_scale, positions, group_size)
+    finally:
+        last = None if pending is None else pending.wait()
+    if last is None:
+        last = int(positions.max().item())
+    cache.length = max(cache.length, last + 1)
 
 
 def _decode_attention_mask(attention_mask: torch.Tensor | None, batch: int, seq_len: int,
@@ -142,6 +149,9 @@ def _decode_attention_mask(attention_mask: torch.Tensor | None, batch: int, seq_
         return bias.masked_fill(rows.logical_not(), -float("inf")).contiguous()
     if attention_mask.dim() == 2:
         cols = attention_mask[:, -seq_len:].to(device=device)
+        bias = _abi.keep_mask_bias(cols, batch, seq_len, device) if cols.is_cuda else None
+        if bias is not None:
+            return bias
         keep = cols if cols.dtype == torch.bool else cols != 0
         bias = torch.zeros((batch, 1, 1, seq_len), device=device, dtype=torch.float32)
         return bias.masked_fill(keep.logical_not()[:, None, None, :], -float("inf"))
@@ -222,18 +232,27 @@ def _forward_fused_int4_kv(self, hidden_states, attention_mask=None, position_id
     def heads(proj, n):
         return proj(hidden_states).view(bsz, q_len, n, self.head_dim).transpose(1, 2).contiguous()
 
-    query_states = heads(self.q_proj, self.num_heads)
-    key_states = heads(self.k_proj, self.num_key_value_heads)
-    value_states = heads(self.v_proj, self.num_key_value_heads)
+    # the step's last position is read back while the projections run (where the position tensor
+    # is used as it is): read after them, it waited for them with the GPU idle behind it
+    pending = None
+    if cache_position is not None and cache_position.device == hidden_states.device \
+            and cache_position.numel() == q_len:
+        pending = _abi.start_max_position(cache_position)
+    try:
+        query_states = heads(self.q_proj, self.num_heads)
+        key_states = heads(self.k_proj, self.num_key_value_heads)
+        value_states = heads(self.v_proj, self.num_key_value_heads)
 
-    group_size = self._int4_kv_group_size
-    if self.head_dim % group_size != 0:
-        raise ValueError(f"head_dim={self.head_dim} must be divisible by group_size={group_size}")
-    if group_size % 2 != 0:
-        raise ValueError(f"group_size={group_size} must be even for INT4 packing")
-
-    positions = _positions(cache_position, q_len, hidden_states.device)
-    required_len = int(positions.max().item()) + 1
+        group_size = self._int4_kv_group_size
+        if self.head_dim % group_size != 0:
+            raise ValueError(
+                f"head_dim={self.head_dim} must be divisible by group_size={group_size}")
+        if group_size % 2 != 0:
+            raise ValueError(f"group_size={group_size} must be even for INT4 packing")
+        positions = _positions(cache_position, q_len, hidden_states.device)
+    finally:
+        last = None if pending is None else pending.wait()
+    required_len = (int(positions.max().item()) if last is None else last) + 1
     layer_cache = _ensure_layer_cache(past_key_value, self.layer_idx, bsz,
                                       self.num_key_value_heads, required_len, self.head_dim,
                                       group_size, hidden_states.device)
@@ -245,7 +264,9 @@ def _forward_fused_int4_kv(self, hidden_states, attention_mask=None, position_id
         attn = attn.reshape(bsz, q_len, self.hidden_size)
         return self.o_proj(attn), None, past_key_value
 
-    _pack_kv_into_cache(layer_cache, key_states, value_states, positions, group_size)
+    _abi.int4_pack_kv_pair(key_states, value_states, layer_cache.k_packed, layer_cache.v_packed,
+                           layer_cache.k_scale, layer_cache.v_scale, positions, group_size)
+    layer_cache.length = max(layer_cache.length, required_len)
 
     key_full = self._int4_kv_repeat_kv(key_states, self.num_key_value_groups)
     value_full = self._int4_kv_repeat_kv(value_states, self.num_key_value_groups)
