@@ -31,6 +31,10 @@
 //     lo the fp32 remainder rounded to fp16), vmax_m the power of two at or above the largest V scale of group m over the
 //     workgroup's keys (one pre-pass over the scales), so P'_m <= 2^8 never overflows fp16; the
 //     output tiles of group m are multiplied by vmax_m at the end.
+// The query rows are read and the 16-bit output rows written 16 bytes at a time where their layout
+// allows (the output through LDS): with 64 element loads and 64 two-byte stores per lane, each
+// behind its own address and dtype branch, a workgroup spent about 10 us outside its tile steps
+// (batch 1, L = 100: 23.2 -> 14.0 us; batch 4, L = 1000, g 128 107 -> 68.6 us; L = 8192 1040 -> 1023 us).
 // Softmax runs in the exp2 domain with a lazily moved running max (rescale only when a score
 // exceeds it by more than 8, so p <= 2^8), as in the decode kernel.
 #include <math.h>
@@ -53,6 +57,7 @@ constexpr int QW = 32;       // query positions per wave (two 16-column tiles)
 constexpr int NW = 4;        // waves per workgroup
 constexpr int KROW = PD + 8; // bf16 per key row of the K tile (272 B: rows 4 banks apart)
 constexpr int VROW = KT + 8; // bf16 per dim row of the V^T tile (80 B)
+constexpr int OROW = PD + 8; // 16-bit values per staged output row (272 B)
 constexpr float LAZY = 8.0f; // running-max slack of the lazy rescale (p <= 2^LAZY)
 constexpr int PG_MAX_D = 512;
 
@@ -103,7 +108,21 @@ struct alignas(16) PrefillLds {
   float ks[2][G][KT];
   float vs[2][G][KT];
   uint16_t vp[2][G][KT];  // vs as fp16, in the P V B-operand order (vpair_slot)
-  float vred[NW][G];
+};
+
+// The state of one column tile that a wave hands to the other key group: o, l and m.
+struct alignas(16) Handover {
+  f32x4_t o[8][64];
+  float l[64], m[64];
+};
+
+// Shared memory of a workgroup of KS key groups: each group's tiles, or (after the key loop) the
+// handed-over states of its waves.
+template <int G, int KS>
+union PrefillShared {
+  PrefillLds<G> tiles[KS];
+  Handover hand[KS == 1 ? 1 : KS * NW];
+  uint16_t rows[KS * NW][QW][OROW];
 };
 
 // One thread's share of a tile's global reads: 8 bytes of K (key tid/8, dwords 2u, 2u+1),
@@ -184,16 +203,58 @@ __device__ __forceinline__ void stage_tile(PrefillLds<G>& s, int nb, const RawTi
   }
 }
 
-template <int G>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+// The bf16 bits of dims 32c + 8 j4 .. + 7 (c = 0 .. 3) of the query row at element `base`, two dims
+// per word: one 16-byte load per c (QV: contiguous head_dim, 16-byte aligned rows), else element
+// loads.
+template <bool QV>
+__device__ __forceinline__ void load_query(const View& q, int64_t base, int j4,
+                                           uint32_t (&w)[4][4]) {
+  const uint16_t* row = (const uint16_t*)q.data + base;
+  if constexpr (QV) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const u32x4_t v = *(const u32x4_t*)(row + 32 * c + 8 * j4);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[c][u] = v[u];
+    }
+  } else {
+    uint32_t e[4][8];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) e[c][u] = row[(32 * c + 8 * j4 + u) * q.s[3]];
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[c][u] = e[c][2 * u] | (e[c][2 * u + 1] << 16);
+    }
+  }
+}
+
+__device__ __forceinline__ uint32_t out_bits(float v, int dtype) {
+  return dtype == LQ_BF16 ? float_to_bf16_bits(v) : __builtin_bit_cast(uint16_t, (_Float16)v);
+}
+
+// KS key groups of NW waves: group kg takes the tiles kg, kg + KS, ... of the workgroup's keys, each
+// group staging its own; with KS = 2 wave w of both groups holds the same query rows, and at the end
+// each hands the other one of its two column tiles and finishes the other (launch_mfma's rule says
+// when that pays). QV and OV: the query and output rows take 16-byte accesses.
+template <int G, int KS, bool QV, bool OV>
+__global__ __launch_bounds__(64 * NW * KS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void prefill_mfma_kernel(PrefillParams p) {
   constexpr int CPG = 4 / G;  // 32-dim chunks per group
   constexpr int NT = 8 / G;   // 16-dim output tiles per group
-  __shared__ PrefillLds<G> lds;
+  constexpr int THREADS = 64 * NW * KS;
+  __shared__ PrefillShared<G, KS> shared;
+  __shared__ float vred[NW * KS][G];
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = threadIdx.x & 63;
+  const int wave_all = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int wave = wave_all % NW;
+  const int kg = wave_all / NW;          // key group
+  const int tid = threadIdx.x % (64 * NW);  // thread of the key group
+  PrefillLds<G>& lds = shared.tiles[kg];
   const int j4 = lane >> 4;
   const int c16 = lane & 15;
   const int L = p.L;
@@ -221,8 +282,18 @@ void prefill_mfma_kernel(PrefillParams p) {
   const float* ksb = p.ks + b * p.kss[0] + kvh * p.kss[1];
   const float* vsb = p.vs + b * p.vss[0] + kvh * p.vss[1];
 
+  // The query rows' bits go out first, so that they return while the V scales are searched. Every
+  // lane loads from a valid row (position clamped to L - 1) and masks afterwards.
+  uint32_t qbits[2][4][4];
+#pragma unroll
+  for (int qt = 0; qt < 2; ++qt) {
+    const int pos = min(q0 + 16 * qt + c16, L - 1);
+    load_query<QV>(p.q, b * p.q.s[0] + (int64_t)head * p.q.s[1] + (int64_t)pos * p.q.s[2], j4,
+                   qbits[qt]);
+  }
+
   RawTile raw;
-  load_tile<G>(kb, vb, ksb, vsb, L, 0, tid, raw);
+  load_tile<G>(kb, vb, ksb, vsb, L, kg * KT, tid, raw);
 
   // vmax_m: power of two at or above the largest V scale of group m over keys [0, gend)
   float vpow[G], vinv[G];
@@ -233,13 +304,13 @@ void prefill_mfma_kernel(PrefillParams p) {
     // eight keys' scales in flight per thread: one key per iteration waited out a full memory
     // round trip each time (64 of them for a workgroup at the end of a 16K-token prompt)
     constexpr int PRE = 8;
-    int k = tid;
-    for (; k + (PRE - 1) * 256 < gend; k += PRE * 256) {
+    int k = threadIdx.x;
+    for (; k + (PRE - 1) * THREADS < gend; k += PRE * THREADS) {
       float v[PRE][G];
 #pragma unroll
       for (int u = 0; u < PRE; ++u) {
 #pragma unroll
-        for (int m = 0; m < G; ++m) v[u][m] = vsb[(int64_t)(k + u * 256) * G + m];
+        for (int m = 0; m < G; ++m) v[u][m] = vsb[(int64_t)(k + u * THREADS) * G + m];
       }
 #pragma unroll
       for (int u = 0; u < PRE; ++u) {
@@ -247,21 +318,21 @@ void prefill_mfma_kernel(PrefillParams p) {
         for (int m = 0; m < G; ++m) mx[m] = fmaxf(mx[m], v[u][m]);
       }
     }
-    for (; k < gend; k += 256) {
+    for (; k < gend; k += THREADS) {
 #pragma unroll
       for (int m = 0; m < G; ++m) mx[m] = fmaxf(mx[m], vsb[(int64_t)k * G + m]);
     }
 #pragma unroll
     for (int m = 0; m < G; ++m) {
       const float w = group_max<64>(mx[m]);
-      if (lane == 0) lds.vred[wave][m] = w;
+      if (lane == 0) vred[wave_all][m] = w;
     }
     __syncthreads();
 #pragma unroll
     for (int m = 0; m < G; ++m) {
-      float v = lds.vred[0][m];
+      float v = vred[0][m];
 #pragma unroll
-      for (int w = 1; w < NW; ++w) v = fmaxf(v, lds.vred[w][m]);
+      for (int w = 1; w < NW * KS; ++w) v = fmaxf(v, vred[w][m]);
       const uint32_t bits = __float_as_uint(v);
       const int e = (int)((bits >> 23) & 0xffu) - 127 + ((bits & 0x7fffffu) != 0 ? 1 : 0);
       const bool ok = v > 0.0f && e > -120 && e < 120;  // normal, finite scales
@@ -270,45 +341,38 @@ void prefill_mfma_kernel(PrefillParams p) {
     }
   }
   stage_tile<G>(lds, 0, raw, tid, p.scale_sm, vinv);
-  if (nsteps > 1) load_tile<G>(kb, vb, ksb, vsb, L, KT, tid, raw);
+  if (nsteps > KS) load_tile<G>(kb, vb, ksb, vsb, L, (KS + kg) * KT, tid, raw);
 
   // Query operands: lane (j4, c16) of column tile qt holds position q0 + 16 qt + c16, dims
   // 32c + 8 j4 + (0,4,1,5,2,6,3,7) for chunk c, as fp16 q * 2^-e with 2^e (qsc) chosen per row
   // so that max |q| * 2^-e lies in [2^14, 2^15).
   u32x4_t qop[2][4];
   float qsc[2];
-  {
-    const uint16_t* qbits = (const uint16_t*)p.q.data;
 #pragma unroll
-    for (int qt = 0; qt < 2; ++qt) {
-      const int pos = q0 + 16 * qt + c16;
-      const bool ok = active && pos < L;
-      // every lane loads from a valid row (position clamped to L - 1) and masks afterwards: a load
-      // under `ok` became a branch with its own wait, 64 round trips in a row per wave
-      const int64_t base =
-          b * p.q.s[0] + (int64_t)head * p.q.s[1] + (int64_t)min(pos, L - 1) * p.q.s[2];
-      float qv[4][8];
-      float mx = 0.0f;
+  for (int qt = 0; qt < 2; ++qt) {
+    const bool ok = active && q0 + 16 * qt + c16 < L;
+    float qv[4][8];
+    float mx = 0.0f;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
+    for (int c = 0; c < 4; ++c) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const float x = bf16_bits_to_float(qbits[base + (32 * c + 8 * j4 + u) * p.q.s[3]]);
-          qv[c][u] = ok ? x : 0.0f;
-          mx = fmaxf(mx, fabsf(qv[c][u]));
-        }
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t w = ok ? qbits[qt][c][u] : 0u;
+        qv[c][2 * u] = __uint_as_float(w << 16);
+        qv[c][2 * u + 1] = __uint_as_float(w & 0xffff0000u);
+        mx = fmaxf(mx, fmaxf(fabsf(qv[c][2 * u]), fabsf(qv[c][2 * u + 1])));
       }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      int e = mx > 0.0f ? (int)((__float_as_uint(mx) >> 23) & 0xffu) - 127 - 14 : 0;
-      e = max(-100, min(100, e));
-      qsc[qt] = __uint_as_float((uint32_t)(127 + e) << 23);
-      const float qinv = __uint_as_float((uint32_t)(127 - e) << 23);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    int e = mx > 0.0f ? (int)((__float_as_uint(mx) >> 23) & 0xffu) - 127 - 14 : 0;
+    e = max(-100, min(100, e));
+    qsc[qt] = __uint_as_float((uint32_t)(127 + e) << 23);
+    const float qinv = __uint_as_float((uint32_t)(127 - e) << 23);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
+    for (int c = 0; c < 4; ++c) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) qop[qt][c][u] = pack_f16(qv[c][u] * qinv, qv[c][u + 4] * qinv);
-      }
+      for (int u = 0; u < 4; ++u) qop[qt][c][u] = pack_f16(qv[c][u] * qinv, qv[c][u + 4] * qinv);
     }
   }
 
@@ -321,15 +385,16 @@ void prefill_mfma_kernel(PrefillParams p) {
     for (int i = 0; i < 8; ++i) o[qt][i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
   }
 
-  for (int st = 0; st < nsteps; ++st) {
-    __syncthreads();  // tile st is staged; the other buffer is free
-    if (st + 1 < nsteps) {
-      stage_tile<G>(lds, (st + 1) & 1, raw, tid, p.scale_sm, vinv);
-      if (st + 2 < nsteps) load_tile<G>(kb, vb, ksb, vsb, L, (st + 2) * KT, tid, raw);
+  // (a key group past the last tile stages zeros from beyond key L and skips them: tb >= wend)
+  for (int st = 0; st < nsteps; st += KS) {
+    const int nb = (st / KS) & 1;
+    __syncthreads();  // this step's tiles are staged; the other buffers are free
+    if (st + KS < nsteps) {
+      stage_tile<G>(lds, nb ^ 1, raw, tid, p.scale_sm, vinv);
+      if (st + 2 * KS < nsteps) load_tile<G>(kb, vb, ksb, vsb, L, (st + 2 * KS + kg) * KT, tid, raw);
     }
-    const int tb = st * KT;
+    const int tb = (st + kg) * KT;
     if (!active || tb >= wend) continue;
-    const int nb = st & 1;
 
     // ---- scores S^T[key][query]: lane holds keys tb + 16t + 4 j4 + r of query column c16
     u32x4_t ka[2][4];
@@ -456,21 +521,86 @@ void prefill_mfma_kernel(PrefillParams p) {
     __builtin_amdgcn_s_setprio(0);
   }
 
-  if (!active) return;
+  if constexpr (KS == 2) {
+    // Group 0 finishes column tile 0, group 1 tile 1: each writes the other's tile of its state to
+    // LDS (over the tiles, read for the last time) and merges what it gets into its own. A group
+    // without a tile has m = -inf, l = 0, o = 0.
+    __syncthreads();
+    Handover& out_h = shared.hand[(1 - kg) * NW + wave];
+    const int send = 1 - kg;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) out_h.o[i][lane] = kg == 0 ? o[1][i] : o[0][i];
+    out_h.l[lane] = l_run[send];
+    out_h.m[lane] = m_run[send];
+    __syncthreads();
+    const Handover& in_h = shared.hand[kg * NW + wave];
+    const float m_own = kg == 0 ? m_run[0] : m_run[1];
+    const float m_in = in_h.m[lane];
+    const float m_new = fmaxf(m_own, m_in);
+    const float a_own = m_own == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_own - m_new);
+    const float a_in = m_in == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_in - m_new);
+    const float l_own = kg == 0 ? l_run[0] : l_run[1];
+    l_run[0] = l_run[1] = l_own * a_own + in_h.l[lane] * a_in;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const f32x4_t v = (kg == 0 ? o[0][i] : o[1][i]) * a_own + in_h.o[i][lane] * a_in;
+      o[0][i] = v;
+      o[1][i] = v;
+    }
+  }
+  __syncthreads();  // the tiles (and handed-over states) were read for the last time
+  float inv[2];
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
     float l = l_run[qt];
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
-    const float inv = 1.0f / l;
+    inv[qt] = 1.0f / l;
+  }
+  if (!active) return;
+  const int64_t obase0 = b * p.out.s[0] + (int64_t)head * p.out.s[1] + (int64_t)q0 * p.out.s[2];
+  if constexpr (OV) {
+    // 16-bit output rows through LDS (the wave's own part), so that 16 lanes store a row of 256
+    // bytes: from the accumulators each store would write 2 bytes of every row
+    uint16_t(&rows)[QW][OROW] = shared.rows[wave_all];
+#pragma unroll
+    for (int qt = 0; qt < 2; ++qt) {
+      if (KS == 2 && qt != kg) continue;
+#pragma unroll
+      for (int it = 0; it < 8; ++it) {
+        uint32_t h[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          h[r] = out_bits(o[qt][it][r] * (vpow[it / NT] * inv[qt]), p.out.dtype);
+        }
+        *(uint2*)&rows[16 * qt + c16][16 * it + 4 * j4] =
+            make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+    const int qs = KS == 2 ? 16 * kg : 0;          // rows qs .. qs + nq - 1
+    constexpr int nq = KS == 2 ? 16 : QW;
+#pragma unroll
+    for (int i = 0; i < nq / 4; ++i) {
+      const int row_i = qs + 4 * i + j4;
+      const u32x4_t v = *(const u32x4_t*)&rows[row_i][8 * c16];
+      if (q0 + row_i < L) {
+        *(u32x4_t*)((uint16_t*)p.out.data + obase0 + (int64_t)row_i * p.out.s[2] + 8 * c16) = v;
+      }
+    }
+    return;
+  }
+#pragma unroll
+  for (int qt = 0; qt < 2; ++qt) {
+    if (KS == 2 && qt != kg) continue;
     const int pos = q0 + 16 * qt + c16;
     if (pos >= L) continue;
-    const int64_t obase = b * p.out.s[0] + (int64_t)head * p.out.s[1] + (int64_t)pos * p.out.s[2];
+    const int64_t obase = obase0 + (int64_t)(16 * qt + c16) * p.out.s[2];
 #pragma unroll
     for (int it = 0; it < 8; ++it) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float v = o[qt][it][r] * (vpow[it / NT] * inv);
+        const float v = o[qt][it][r] * (vpow[it / NT] * inv[qt]);
         store_float(p.out.data, p.out.dtype, obase + (int64_t)(16 * it + 4 * j4 + r) * p.out.s[3], v);
       }
     }
@@ -576,20 +706,56 @@ bool prefill_mfma_ok(const PrefillParams& p) {
   return true;
 }
 
+// 16-bit rows along head_dim, contiguous and 16-byte aligned.
+bool rows_aligned(const View& v) {
+  return v.s[3] == 1 && ((uintptr_t)v.data & 15) == 0 && v.s[0] % 8 == 0 && v.s[1] % 8 == 0 &&
+         v.s[2] % 8 == 0;
+}
+
 // Workgroup order: the units vary fastest, so the heaviest position block of every (batch, KV head)
 // launches first and the lightest blocks fill the end, and with 8 units each XCD keeps one head's
 // K and V in its L2. With the position blocks fastest, the last unit's heaviest blocks started
 // when the others were done: batch 1, 8 KV heads, L = 4096 442 -> 296 us, 8192 1278 -> 1060 us,
 // 16384 4143 -> 3970 us; batch 2, L = 777 63.7 -> 56.0 us. (More than 65535 position blocks do not
 // fit grid.y and keep the position blocks in grid.x.)
+//
+// Two key groups (KS = 2) while every workgroup finds a slot of two per CU anyway (256 CUs): the
+// time is then that of the longest chain of tile steps, which two groups halve. L = 777, batch 2
+// 43.0 -> 37.4 us; batch 1, L = 500 32.2 -> 26.5, 1024 57.0 -> 44.3, 1500 72.0 -> 52.2, 2048 (512
+// workgroups) 112.6 -> 91.5 us. With more workgroups the independent four-wave ones are faster
+// (their waves are in different phases of a step): batch 4, L = 600 (608 workgroups) 42.4 against
+// 56.2 us, batch 1, L = 3000 165 against 194, 8192 1023 against 1165 us.
+constexpr int64_t KS2_WORKGROUPS = 512;
+
+template <int G, int KS>
+void launch_mfma_ks(const PrefillParams& p, dim3 grid, hipStream_t st) {
+  const bool qv = rows_aligned(p.q);
+  const bool ov = p.out.dtype != LQ_F32 && rows_aligned(p.out);
+  const dim3 block(64 * NW * KS);
+  if (qv && ov) {
+    hipLaunchKernelGGL((prefill_mfma_kernel<G, KS, true, true>), grid, block, 0, st, p);
+  } else if (qv) {
+    hipLaunchKernelGGL((prefill_mfma_kernel<G, KS, true, false>), grid, block, 0, st, p);
+  } else if (ov) {
+    hipLaunchKernelGGL((prefill_mfma_kernel<G, KS, false, true>), grid, block, 0, st, p);
+  } else {
+    hipLaunchKernelGGL((prefill_mfma_kernel<G, KS, false, false>), grid, block, 0, st, p);
+  }
+}
+
 template <int G>
 void launch_mfma(PrefillParams p, hipStream_t st) {
   const int64_t npb = ((int64_t)p.L + QW - 1) / QW;
   const int64_t nwg = (npb * p.nrep + NW - 1) / NW;
-  const unsigned units = (unsigned)(p.B * p.Hkv);
+  const int64_t units = (int64_t)p.B * p.Hkv;
   p.unit_fast = nwg <= 65535;
-  const dim3 grid = p.unit_fast ? dim3(units, (unsigned)nwg) : dim3((unsigned)nwg, units);
-  hipLaunchKernelGGL((prefill_mfma_kernel<G>), grid, dim3(256), 0, st, p);
+  const dim3 grid = p.unit_fast ? dim3((unsigned)units, (unsigned)nwg)
+                                : dim3((unsigned)nwg, (unsigned)units);
+  if (nwg * units <= KS2_WORKGROUPS) {
+    launch_mfma_ks<G, 2>(p, grid, st);
+  } else {
+    launch_mfma_ks<G, 1>(p, grid, st);
+  }
 }
 
 }  // namespace
