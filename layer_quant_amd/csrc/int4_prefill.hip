@@ -128,33 +128,33 @@ union PrefillShared {
 // One thread's share of a tile's global reads: 8 bytes of K (key tid/8, dwords 2u, 2u+1),
 // dword tid/16 of the V rows of keys 2(tid%16), 2(tid%16)+1 (consecutive lanes take consecutive
 // key pairs, so the transposed LDS writes of a wave fill whole rows instead of hitting one bank
-// per row 8 apart), and one scale word (K scales on threads 0..127, V scales on 128..255). Keys
-// at or past L read as zero.
+// per row 8 apart), and one scale word (K scales on threads 0..127, V scales on 128..255).
 struct RawTile {
   uint32_t k0, k1;
   uint32_t v0, v1;
   float sc;
 };
 
+// (Rows past L - 1 read row L - 1 again: a query below L gives them p = 0, as it gives the rows
+// between it and L. A tile's base is uniform and the lane offsets are 32-bit.)
 template <int G>
 __device__ __forceinline__ void load_tile(const uint8_t* kb, const uint8_t* vb, const float* ksb,
                                           const float* vsb, int L, int tb, int tid, RawTile& r) {
-  const int kk = tb + (tid >> 3);
-  if (kk < L) {
-    const uint2 w = *(const uint2*)(kb + (int64_t)kk * 64 + 8 * (tid & 7));
-    r.k0 = w.x;
-    r.k1 = w.y;
-  } else {
-    r.k0 = 0;
-    r.k1 = 0;
-  }
-  const int vk = tb + 2 * (tid & 15);
-  r.v0 = vk < L ? *(const uint32_t*)(vb + (int64_t)vk * 64 + 4 * (tid >> 4)) : 0u;
-  r.v1 = vk + 1 < L ? *(const uint32_t*)(vb + (int64_t)(vk + 1) * 64 + 4 * (tid >> 4)) : 0u;
-  const int si = tid & 127;
-  const int sk = tb + (si & (KT - 1));  // scale word (key si % 32, group si / 32)
-  const float* sb = tid < 128 ? ksb : vsb;
-  r.sc = (si < G * KT && sk < L) ? sb[(int64_t)sk * G + (si / KT)] : 0.0f;
+  tb = min(tb, (L - 1) & ~(KT - 1));
+  const int last = L - 1 - tb;  // >= 0
+  const uint8_t* kt = kb + (int64_t)tb * 64;
+  const uint8_t* vt = vb + (int64_t)tb * 64;
+  const uint32_t kk = min(tid >> 3, last);
+  const uint2 w = *(const uint2*)(kt + (kk * 64u + 8u * (tid & 7)));
+  r.k0 = w.x;
+  r.k1 = w.y;
+  const uint32_t v0 = min(2 * (tid & 15), last), v1 = min(2 * (tid & 15) + 1, last);
+  r.v0 = *(const uint32_t*)(vt + (v0 * 64u + 4u * (tid >> 4)));
+  r.v1 = *(const uint32_t*)(vt + (v1 * 64u + 4u * (tid >> 4)));
+  // scale word (key si % 32, group si / 32); the threads past G * KT read the first ones again
+  const int si = tid & (G * KT - 1);
+  const float* sb = (tid < 128 ? ksb : vsb) + (int64_t)tb * G;
+  r.sc = sb[(uint32_t)min(si & (KT - 1), last) * G + si / KT];
 }
 
 // key k of a tile -> its half-word in the fp16 V-scale row: lane group j's B-operand key pairs
