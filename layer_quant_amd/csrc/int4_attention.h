@@ -32,6 +32,9 @@ struct AttnParams {
   // [B, Hkv, D] (strides of b, h, d) are packed into cache row S - 1 inside the kernel
   View knew, vnew;
   int pack;
+  int q_rows;    // MFMA path: query rows contiguous and 4-byte aligned (loaded to LDS directly)
+  int tok_rows;  // the same for the new token's rows, of a 16-bit type
+  int grid3;     // MFMA path: grid (KV heads, batch, splits) instead of (units, splits)
 };
 
 struct SplitPlan {

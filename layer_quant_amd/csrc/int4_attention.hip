@@ -152,7 +152,7 @@ __device__ __forceinline__ float wave_sum(float v) {
 // the splits s = g mod G (G = 256 / D split groups for D <= 256; each thread takes two dims of one
 // group for larger D), and the group partials are summed through LDS.
 constexpr int MERGE_THREADS = 256;
-constexpr int MERGE_SPT = 16;  // splits per thread of the one-round-trip merge
+constexpr int MERGE_PER_GROUP = 16, MERGE_GROUPS = 4;  // attn_merge_few_kernel: up to 64 splits
 
 __device__ __forceinline__ float block_reduce(float v, bool is_max, float* red) {
   v = is_max ? wave_max(v) : wave_sum(v);
@@ -181,47 +181,6 @@ __global__ __launch_bounds__(MERGE_THREADS) void attn_merge_kernel(AttnParams p)
   const int g = tid / dw;
   const int d0 = tid - g * dw;
   const int64_t obase = b * p.out.s[0] + qh * p.out.s[1];
-  if (D <= MERGE_THREADS && ns <= groups * MERGE_SPT && ns <= MERGE_THREADS) {
-    // One memory round trip: every load this thread needs (its acc partials of dim d0 over the
-    // splits g, g + groups, ..., their m, and one (m, l) pair for the block reductions) goes out
-    // before the first use; addresses are clamped to valid splits and the extra values masked.
-    // The same sums in the same order as the loop form below, so the results are identical. In
-    // the kernel trace the merge took 4.16 against 4.36 us (median over batch 1 and 8, 5-32
-    // splits): most of a merge launch is the launch itself.
-    float pa[MERGE_SPT], pm[MERGE_SPT];
-    const int gc = min(g, groups - 1);
-#pragma unroll
-    for (int i = 0; i < MERGE_SPT; ++i) {
-      const int sc = min(gc + i * groups, ns - 1);
-      pa[i] = p.ws_acc[(base + sc) * D + d0];
-      pm[i] = p.ws_m[base + sc];
-    }
-    const int tc = min(tid, ns - 1);
-    const float mt0 = p.ws_m[base + tc];
-    const float lt0 = p.ws_l[base + tc];
-    const float mt = tid < ns ? mt0 : -INFINITY;
-    const float M = block_reduce(mt, true, red);
-    const float L =
-        block_reduce((mt == -INFINITY) ? 0.0f : exp2f(mt - M) * lt0, false, red);
-    float acc = 0.0f;
-#pragma unroll
-    for (int i = 0; i < MERGE_SPT; ++i) {
-      const int s = g + i * groups;
-      if (g < groups && s < ns) {
-        const float w = (pm[i] == -INFINITY) ? 0.0f : exp2f(pm[i] - M);
-        acc += w * pa[i];
-      }
-    }
-    if (groups > 1) {
-      part[tid] = acc;
-      __syncthreads();
-      if (g == 0) {
-        for (int i = 1; i < groups; ++i) acc += part[i * dw + d0];
-      }
-    }
-    if (g == 0) store_float(p.out.data, p.out.dtype, obase + d0 * p.out.s[2], acc / L);
-    return;
-  }
   float M = -INFINITY;
   for (int s = tid; s < ns; s += MERGE_THREADS) M = fmaxf(M, p.ws_m[base + s]);
   M = block_reduce(M, true, red);
@@ -254,6 +213,86 @@ __global__ __launch_bounds__(MERGE_THREADS) void attn_merge_kernel(AttnParams p)
     }
     if (g == 0) store_float(p.out.data, p.out.dtype, obase + d * p.out.s[2], acc / L);
   }
+}
+
+// The same for at most NS * groups splits and D <= 256: thread d of each group of blockDim.x / groups
+// threads holds dim d of one (batch, query head) over the splits g, g + groups, ... Its partials and
+// the splits' m and l (the same for every lane of a wave: scalar loads) all go out at once, and every
+// lane makes the weights itself: one memory round trip and no reduction across lanes; more than one
+// group joins through LDS. With two block reductions before the weights (attn_merge_kernel) the launch
+// took 3.9 us in the kernel trace at 8 splits, batch 1, and 4.4 at 32; here 2.9 and 3.9 us. (All of
+// 32 splits in one thread: 8.8 us.)
+template <int NS>
+__global__ __launch_bounds__(1024) void attn_merge_few_kernel(const float* __restrict__ ws_m,
+                                                              const float* __restrict__ ws_l,
+                                                              const float* __restrict__ ws_acc,
+                                                              View out, int Hq, int D, int ns,
+                                                              int groups) {
+  __shared__ float s_acc[1024], s_m[MERGE_GROUPS], s_l[MERGE_GROUPS];
+  const int bh = blockIdx.x;
+  const int64_t base = (int64_t)bh * ns;
+  const int width = (int)blockDim.x / groups;  // D rounded up to whole waves
+  const int g = __builtin_amdgcn_readfirstlane((int)threadIdx.x / width);
+  const int t = (int)threadIdx.x - g * width;
+  const int d = min(t, D - 1);
+  float part[NS], m[NS], l[NS];
+#pragma unroll
+  for (int i = 0; i < NS; ++i) part[i] = ws_acc[(base + min(g + i * groups, ns - 1)) * D + d];
+#pragma unroll
+  for (int i = 0; i < NS; ++i) {
+    m[i] = ws_m[base + min(g + i * groups, ns - 1)];
+    l[i] = ws_l[base + min(g + i * groups, ns - 1)];
+  }
+  float M = m[0];  // (a repeated last split changes no maximum; its weight below is 0)
+#pragma unroll
+  for (int i = 1; i < NS; ++i) M = fmaxf(M, m[i]);
+  float L = 0.0f, acc = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NS; ++i) {
+    const bool in = g + i * groups < ns && m[i] != -INFINITY;
+    const float w = in ? __builtin_amdgcn_exp2f(m[i] - M) : 0.0f;
+    L += w * l[i];
+    acc += w * part[i];
+  }
+  if (groups > 1) {
+    s_acc[threadIdx.x] = acc;
+    if (t == 0) {
+      s_m[g] = M;
+      s_l[g] = L;
+    }
+    __syncthreads();
+    if (g > 0) return;
+    float Mt = s_m[0];
+    for (int i = 1; i < groups; ++i) Mt = fmaxf(Mt, s_m[i]);
+    L = acc = 0.0f;
+    for (int i = 0; i < groups; ++i) {
+      const float w = s_m[i] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(s_m[i] - Mt);
+      L += w * s_l[i];
+      acc += w * s_acc[i * width + t];
+    }
+  }
+  if (t >= D) return;
+  const int b = bh / Hq;
+  const int qh = bh - b * Hq;
+  store_float(out.data, out.dtype, b * out.s[0] + qh * out.s[1] + d * out.s[2], acc / L);
+}
+
+static void launch_merge(const AttnParams& p, hipStream_t st) {
+  const dim3 grid((unsigned)(p.B * p.Hq));
+  const int groups = (p.nsplit + MERGE_PER_GROUP - 1) / MERGE_PER_GROUP;
+  if (p.D > 256 || groups > MERGE_GROUPS) {
+    hipLaunchKernelGGL(attn_merge_kernel, grid, dim3(MERGE_THREADS), 0, st, p);
+    return;
+  }
+  const int per = (p.nsplit + groups - 1) / groups;
+  const dim3 block((unsigned)(groups * ((p.D + 63) / 64 * 64)));
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, st, p.ws_m, p.ws_l, p.ws_acc, p.out, p.Hq, p.D,
+                       p.nsplit, groups);
+  };
+  if (per <= 4) go(attn_merge_few_kernel<4>);
+  else if (per <= 8) go(attn_merge_few_kernel<8>);
+  else go(attn_merge_few_kernel<MERGE_PER_GROUP>);
 }
 
 // Split plan of the generic kernel: about 2048 waves in flight, at least 64 keys per split.
@@ -577,7 +616,7 @@ static int decode_attention(const lq_tensor* q, const lq_tensor* k_packed,
     if ((rc = check_launch("lq_int4_decode_attention")) != LQ_OK) return rc;
   }
   if (p.nsplit > 1 && !p.fold) {
-    hipLaunchKernelGGL(attn_merge_kernel, dim3((unsigned)(B * Hq)), dim3(MERGE_THREADS), 0, st, p);
+    launch_merge(p, st);
     if ((rc = check_launch("lq_int4_decode_attention merge")) != LQ_OK) return rc;
   }
   return LQ_OK;

@@ -347,16 +347,19 @@ __global__ __launch_bounds__(THREADS) void attn_fast_kernel(AttnParams p) {
   __shared__ TileLds tiles1[WAVES];
   __shared__ TileLds tiles2[WAVES];
   __shared__ float o_sep[O_IN_TILE ? 1 : WAVES * (NREP * FAST_D + 2 * NREP)];
+  __shared__ u32x4_t q_lds[WAVES][NREP * FAST_D / 8];  // each wave's copy of the query rows (bf16)
+  __shared__ uint32_t tok_lds[2][FAST_D / 2];          // the new token's K and V rows
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q4 = lane >> 4;
   const int c16 = lane & 15;
-  const int unit = blockIdx.x;
-  const int split = blockIdx.y;
-  const int b = unit / p.Hkv;
-  const int kvh = unit - b * p.Hkv;
+  // (a grid axis each for KV head and batch saves the division before the first load)
+  const int split = p.grid3 ? blockIdx.z : blockIdx.y;
+  const int b = p.grid3 ? blockIdx.y : blockIdx.x / p.Hkv;
+  const int kvh = p.grid3 ? blockIdx.x : blockIdx.x - b * p.Hkv;
+  const int unit = b * p.Hkv + kvh;
   const int S = (int)p.S;
   const int t0 = split * (int)p.chunk;
   const int t1 = min(S, t0 + (int)p.chunk);
@@ -383,35 +386,87 @@ __global__ __launch_bounds__(THREADS) void attn_fast_kernel(AttnParams p) {
   R.msk_bytes = (int)(p.mask_sk * 4);
   R.mask_len = p.mask_len;
 
-  // the first tiles' loads go out before the query set-up
+  // Fused pack (lq_int4_decode_attention_pack): the wave whose dealt tiles hold key S - 1 (its
+  // last tile) loads the new token's K and V rows first (lane j: dims 2j and 2j + 1) and packs them
+  // when it reaches that tile, after the tile's wait (a full one, the last tile having no
+  // loads behind it): the pack kernel's arithmetic, written to cache row S - 1 and over the key's
+  // row in the LDS tile, whichever version the tile's loads read. (The fast path's caches have
+  // 64-byte rows and contiguous scales, so the row is indexed directly.)
+  constexpr int GH = FAST_D / (2 * G);  // lanes per quantisation group
+  int pack_i = -1;                      // the wave's tile index holding key S - 1, or -1
+  const int64_t kx = b * p.knew.s[0] + (int64_t)kvh * p.knew.s[1];
+  const int64_t vx = b * p.vnew.s[0] + (int64_t)kvh * p.vnew.s[1];
+  if (p.pack && t1 == S) {
+    const int tile = (S - 1 - t0) / TILE;
+    if (tile % WAVES == wave) {
+      pack_i = tile / WAVES;
+      if (p.tok_rows) {
+        load_to_lds_b32(make_desc((const uint16_t*)p.knew.data + kx, FAST_D * 2), &tok_lds[0][0], 4 * lane);
+        load_to_lds_b32(make_desc((const uint16_t*)p.vnew.data + vx, FAST_D * 2), &tok_lds[1][0], 4 * lane);
+      }
+    }
+  }
+  // The query rows go out before the first tiles, straight to LDS: 16 bytes per lane, lane l of load
+  // j taking head 4j + l/16, dims 8 (l & 15) .. + 7. Loaded to registers (32 two-byte loads per lane)
+  // they came after the tiles, whose loads the compiler's waits for them then waited for too.
+  // (Kernel trace, with the grid's axes and the plain partial stores: batch 1, ctx 1000 7.1 -> 6.4 us,
+  // ctx 16384 12.2 -> 10.0; batch 8, ctx 2072 11.8 -> 9.3, ctx 4001 15.3 -> 13.7 us.)
+  const int64_t qbase = b * p.q.s[0] + (int64_t)(kvh * NREP) * p.q.s[1];
+  if (p.q_rows) {
+    const i32x4_t rq = make_desc((const uint16_t*)p.q.data + qbase,
+                                 (int)((NREP - 1) * p.q.s[1] * 2) + FAST_D * 2);
+#pragma unroll
+    for (int j = 0; j < (NREP + 3) / 4; ++j) {
+      const int h = 4 * j + q4;
+      if (NREP >= 4 || h < NREP) {
+        load_to_lds(rq, &q_lds[wave][64 * j], h * (int)p.q.s[1] * 2 + 16 * c16);
+      }
+    }
+  }
   if (nw > 0) issue_tile<G, MASK>(R, tile_key(0), S, tiles0[wave], lane);
   if (nw > 1) issue_tile<G, MASK>(R, tile_key(1), S, tiles1[wave], lane);
 
   // Query operands. Lane (q, .) feeds MFMA c with dword c of its key unit q, i.e. dims
-  // 32q + 8c .. 32q + 8c + 7 (slot order kPerm); the query is placed only in the columns whose
+  // 32q + 8c .. 32q + 8c + 7 in slot order (0,4,1,5,2,6,3,7); the query is placed only in the columns whose
   // group owns those dims, so each column accumulates exactly its group's partial dot product.
-  const uint16_t* qbits = (const uint16_t*)p.q.data;
-  const int64_t qbase = b * p.q.s[0] + (int64_t)(kvh * NREP + colh) * p.q.s[1];
-  constexpr int kPerm[8] = {0, 4, 1, 5, 2, 6, 3, 7};
   const bool use = colvalid && (q4 / CPG == colm);
-  // Every lane loads its 32 values (the address is valid for every lane) and the unused ones are
-  // zeroed afterwards: loaded under `use`, each pair became a branch with its own wait.
-  uint32_t qraw[4][8];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) qraw[c][k] = qbits[qbase + (32 * q4 + 8 * c + kPerm[k]) * p.q.s[2]];
-  }
   u32x4_t qop[4];
+  if (p.q_rows) {
+    if (nw > 1) wait_loads<2 * LPT>();
+    else if (nw > 0) wait_loads<LPT>();
+    else wait_loads<0>();
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const u32x4_t w = q_lds[wave][16 * colh + 4 * q4 + c];
+      qop[c][0] = __builtin_amdgcn_perm(w.z, w.x, 0x05040100u);
+      qop[c][1] = __builtin_amdgcn_perm(w.z, w.x, 0x07060302u);
+      qop[c][2] = __builtin_amdgcn_perm(w.w, w.y, 0x05040100u);
+      qop[c][3] = __builtin_amdgcn_perm(w.w, w.y, 0x07060302u);
+    }
+  } else {
+    // Every lane loads its 32 values (the address is valid for every lane) and the unused ones are
+    // zeroed afterwards: loaded under `use`, each pair became a branch with its own wait.
+    constexpr int kPerm[8] = {0, 4, 1, 5, 2, 6, 3, 7};
+    const uint16_t* qbits = (const uint16_t*)p.q.data + qbase + colh * p.q.s[1];
+    uint32_t qraw[4][8];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) qraw[c][k] = qbits[(32 * q4 + 8 * c + kPerm[k]) * p.q.s[2]];
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) qop[c][u] = qraw[c][2 * u] | (qraw[c][2 * u + 1] << 16);
+    }
+  }
   float qsum = 0.0f;
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const uint32_t lo = use ? qraw[c][2 * u] : 0u;
-      const uint32_t hi = use ? qraw[c][2 * u + 1] : 0u;
-      qsum += bf16_bits_to_float(lo) + bf16_bits_to_float(hi);
-      qop[c][u] = lo | (hi << 16);
+      qop[c][u] = use ? qop[c][u] : 0u;
+      qsum += bf16_bits_to_float(qop[c][u]) + __uint_as_float(qop[c][u] & 0xffff0000u);
     }
   }
   qsum += __shfl_xor(qsum, 16, 64);
@@ -420,31 +475,17 @@ __global__ __launch_bounds__(THREADS) void attn_fast_kernel(AttnParams p) {
   const float csm = p.scale_sm;  // raw scores -> log2 units
   const float inv_csm = 1.0f / csm;
 
-  // Fused pack (lq_int4_decode_attention_pack): the wave whose dealt tiles hold key S - 1 (its
-  // last tile) loads the new token's K and V values here (lane j: dims 2j and 2j + 1) and packs
-  // them when it reaches that tile, after the tile's wait (a full one, the last tile having no
-  // loads behind it): the pack kernel's arithmetic, written to cache row S - 1 and over the key's
-  // row in the LDS tile, whichever version the tile's loads read. (The fast path's caches have
-  // 64-byte rows and contiguous scales, so the row is indexed directly.)
-  constexpr int GH = FAST_D / (2 * G);  // lanes per quantisation group
-  int pack_i = -1;                      // the wave's tile index holding key S - 1, or -1
   float kx0 = 0.0f, kx1 = 0.0f, vx0 = 0.0f, vx1 = 0.0f;
-  if (p.pack && t1 == S) {
-    const int tile = (S - 1 - t0) / TILE;
-    if (tile % WAVES == wave) {
-      pack_i = tile / WAVES;
-      const int64_t kx = b * p.knew.s[0] + (int64_t)kvh * p.knew.s[1];
-      const int64_t vx = b * p.vnew.s[0] + (int64_t)kvh * p.vnew.s[1];
-      uint32_t sh[4];
-      const uint32_t w0 = elem_word(p.knew.data, p.knew.dtype, kx + 2 * lane * p.knew.s[2], sh[0]);
-      const uint32_t w1 = elem_word(p.knew.data, p.knew.dtype, kx + (2 * lane + 1) * p.knew.s[2], sh[1]);
-      const uint32_t w2 = elem_word(p.vnew.data, p.vnew.dtype, vx + 2 * lane * p.vnew.s[2], sh[2]);
-      const uint32_t w3 = elem_word(p.vnew.data, p.vnew.dtype, vx + (2 * lane + 1) * p.vnew.s[2], sh[3]);
-      kx0 = word_elem(w0, sh[0], p.knew.dtype);
-      kx1 = word_elem(w1, sh[1], p.knew.dtype);
-      vx0 = word_elem(w2, sh[2], p.vnew.dtype);
-      vx1 = word_elem(w3, sh[3], p.vnew.dtype);
-    }
+  if (pack_i >= 0 && !p.tok_rows) {  // token rows of any strides and type
+    uint32_t sh[4];
+    const uint32_t w0 = elem_word(p.knew.data, p.knew.dtype, kx + 2 * lane * p.knew.s[2], sh[0]);
+    const uint32_t w1 = elem_word(p.knew.data, p.knew.dtype, kx + (2 * lane + 1) * p.knew.s[2], sh[1]);
+    const uint32_t w2 = elem_word(p.vnew.data, p.vnew.dtype, vx + 2 * lane * p.vnew.s[2], sh[2]);
+    const uint32_t w3 = elem_word(p.vnew.data, p.vnew.dtype, vx + (2 * lane + 1) * p.vnew.s[2], sh[3]);
+    kx0 = word_elem(w0, sh[0], p.knew.dtype);
+    kx1 = word_elem(w1, sh[1], p.knew.dtype);
+    vx0 = word_elem(w2, sh[2], p.vnew.dtype);
+    vx1 = word_elem(w3, sh[3], p.vnew.dtype);
   }
 
   // QK A-row i of a 16-key half is key 4 (i & 3) + (i >> 2), so that output row 4q + r (held by
@@ -473,6 +514,13 @@ __global__ __launch_bounds__(THREADS) void attn_fast_kernel(AttnParams p) {
     wait_tile(i);
     if (i == pack_i) {  // key S - 1 of this tile: the fused pack (LDS layout as in TileLds)
       float kscl, vscl;
+      if (p.tok_rows) {
+        const uint32_t kw = tok_lds[0][lane], vw = tok_lds[1][lane];
+        kx0 = word_elem(kw, 0, p.knew.dtype);
+        kx1 = word_elem(kw, 16, p.knew.dtype);
+        vx0 = word_elem(vw, 0, p.vnew.dtype);
+        vx1 = word_elem(vw, 16, p.vnew.dtype);
+      }
       const uint32_t kbyte = int4_quantize_pair<GH>(kx0, kx1, kscl);
       const uint32_t vbyte = int4_quantize_pair<GH>(vx0, vx1, vscl);
       const int key = S - 1 - tb;
@@ -677,7 +725,7 @@ __global__ __launch_bounds__(THREADS) void attn_fast_kernel(AttnParams p) {
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
       const float mw = o_wave(w)[NREP * FAST_D + h];
-      const float wt = (mw == -INFINITY) ? 0.0f : exp2f(mw - M);
+      const float wt = (mw == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(mw - M);
       L += wt * o_wave(w)[NREP * FAST_D + NREP + h];
       a += wt * o_wave(w)[h * FAST_D + d];
     }
@@ -687,10 +735,18 @@ __global__ __launch_bounds__(THREADS) void attn_fast_kernel(AttnParams p) {
                   a / L);
     } else {
       const int64_t slot = ((int64_t)b * p.Hq + qh) * p.nsplit + split;
-      coherent_store(&p.ws_acc[slot * FAST_D + d], a);
-      if (d == 0) {
-        coherent_store(&p.ws_m[slot], M);
-        coherent_store(&p.ws_l[slot], L);
+      if (p.fold) {
+        coherent_store(&p.ws_acc[slot * FAST_D + d], a);
+        if (d == 0) {
+          coherent_store(&p.ws_m[slot], M);
+          coherent_store(&p.ws_l[slot], L);
+        }
+      } else {
+        p.ws_acc[slot * FAST_D + d] = a;
+        if (d == 0) {
+          p.ws_m[slot] = M;
+          p.ws_l[slot] = L;
+        }
       }
     }
   }
@@ -807,9 +863,20 @@ SplitPlan plan_fast(int64_t B, int64_t Hkv, int64_t S) {
   return sp;
 }
 
+// Rows of a 16-bit type that the kernel loads to LDS 4 or 16 bytes per lane: contiguous head_dim,
+// 4-byte aligned, and (for n rows) 32-bit offsets.
+static bool lds_rows_ok(const View& v, int64_t n) {
+  return v.dtype != LQ_F32 && v.s[2] == 1 && ((uintptr_t)v.data & 3) == 0 && v.s[0] % 2 == 0 &&
+         v.s[1] % 2 == 0 && v.s[1] >= 0 && n * v.s[1] * 2 < ((int64_t)1 << 31) - FAST_D * 2;
+}
+
 template <int NREP, int G>
-static void launch_one(const AttnParams& p, hipStream_t st) {
-  const dim3 grid((unsigned)(p.B * p.Hkv), (unsigned)p.nsplit);
+static void launch_one(AttnParams p, hipStream_t st) {
+  p.q_rows = lds_rows_ok(p.q, NREP);
+  p.tok_rows = p.pack && lds_rows_ok(p.knew, 1) && lds_rows_ok(p.vnew, 1);
+  p.grid3 = p.B <= 65535 && p.nsplit <= 65535;
+  const dim3 grid = p.grid3 ? dim3((unsigned)p.Hkv, (unsigned)p.B, (unsigned)p.nsplit)
+                            : dim3((unsigned)(p.B * p.Hkv), (unsigned)p.nsplit);
   if (p.mask != nullptr) {
     hipLaunchKernelGGL((attn_fast_kernel<NREP, G, true>), grid, dim3(THREADS), 0, st, p);
   } else {
