@@ -725,10 +725,6 @@ __global__ __launch_bounds__(256) void mx_update_kernel(MxUpdateParams p) {
 // Lane offsets are 32-bit offsets into per-(batch, head) buffer descriptors. Same arithmetic as
 // mx_update_kernel in the (B*dt)*x order; in the counter mode rng_offset is a multiple of 16, so a
 // block's pair counters are lo0 | k and lowbias32's first step folds into one per-block word.
-#ifndef LQ_MX_ROWS_WAVES
-#define LQ_MX_ROWS_WAVES 1
-#endif
-
 // State blocks and x words of R rows of one lane (the raw loads of one work item).
 template <int R>
 struct RowLoads {
@@ -799,11 +795,10 @@ __device__ __forceinline__ void load_rows(const MxUpdateParams& p, const HeadBuf
 }
 
 // Update, y, and writeback encode of the R rows held in L. bdp and cvp point to the lane's 16
-// values of B * dt and C in LDS, read again for every row instead of once into 32 VGPRs: the
-// compact layouts' 4-row form then fits 74 VGPRs (6 waves per SIMD instead of 5; MX4 at batch 64
-// 38.7 -> 37.1 us, batch 128 72.0 -> 68.1 us on one box), the reference layout's 2-row form 67
-// (7 waves instead of 6; MX4 at batch 64 39.0-39.2 -> 38.3-38.6 us on one box, three alternated
-// runs; with the earlier, VALU-heavier encoder it had been slower, 42.5 against 39.6 us).
+// values of B * dt and C in LDS, read again for every row instead of once into 32 VGPRs: 67 VGPRs
+// in the reference layout (7 waves per SIMD instead of 6; MX4 at batch 64 39.0-39.2 -> 38.3-38.6 us on
+// one box, three alternated runs; with the earlier, VALU-heavier encoder it had been slower, 42.5
+// against 39.6 us).
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 template <int FB, int RMODE, int BPR_LOG2, int R, int SLOTS, int LY>
@@ -926,17 +921,8 @@ __device__ __forceinline__ void update_rows(const MxUpdateParams& p, const HeadB
 // One work item per workgroup: grid (ceil(P / (R * SLOTS)), H, B). Every state load of the lane
 // (R state blocks, x, z) is issued before the first use of any of them; B, C and the head scalars
 // come through LDS (one barrier).
-// The byte-mantissa compact layout (CM8) asks for 6 waves per SIMD: its 4-row form then fits 77-79
-// VGPRs without spills instead of taking 84 (5 waves); MX8 at batch 64, three alternated rounds on
-// one box: 35.71-35.91 against 36.60-37.33 us. Its supplied-uniform form (2 rows, 256 threads)
-// would spill under the cap and keeps the default, as do the other layouts (the nibble layout's
-// MX4 form spills at 6 waves).
-constexpr int rows_waves(int LY, int RMODE) {
-  return LY == LAYOUT_CM8 && RMODE != LQ_ROUND_SR_UNIFORM ? 6 : LQ_MX_ROWS_WAVES;
-}
 template <int FB, int RMODE, int BPR_LOG2, int R, int THREADS, int LY>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(rows_waves(LY, RMODE))))
-void mx_update_rows_kernel(MxUpdateParams p) {
+__global__ __launch_bounds__(THREADS) void mx_update_rows_kernel(MxUpdateParams p) {
   constexpr int BPR = 1 << BPR_LOG2;
   constexpr uint32_t N = 16 * BPR;
   constexpr int SLOTS = THREADS >> BPR_LOG2;
@@ -1322,30 +1308,31 @@ static void dispatch_encode(const MxCodecParams& p, int rmode, bool vec, dim3 gr
 }
 
 // Rows kernel geometry: R rows per lane, THREADS threads, one (batch, head) slice of up to
-// R * THREADS / (N/16) rows per workgroup (64 rows = one Nemotron-H head at N = 128). The reference
-// layout keeps 2 rows per lane (67 VGPRs, 7 waves per SIMD: its 212 MB per call at batch 64 need
-// the waves to hide memory latency; 4 rows per lane take 87 VGPRs, 5 waves, and with an earlier
-// build ran 42.2 against 41.4 us). The compact layouts move 2.5x fewer bytes and are bound by their arithmetic, so 4 rows
-// per lane share the per-lane setup (head scalars, B and C) over twice the rows: 41.1 -> 38.9 us
-// for MX4 at batch 64 (91 VGPRs, 5 waves per SIMD). The supplied-uniform mode keeps 2 rows per
-// lane everywhere: its 16 uniforms per row would take 155-161 VGPRs at 4 rows. So does the Philox
-// mode, whose 4-row form kept the rows' arrays in scratch memory.
-template <int LY, int RMODE>
-struct RowsGeometry {
-  static constexpr bool wide =
-      LY != LAYOUT_REF && RMODE != LQ_ROUND_SR_UNIFORM && RMODE != LQ_ROUND_SR_PHILOX;
-  static constexpr int R = wide ? 4 : 2;
-  static constexpr int THREADS = wide ? 128 : 256;
-  static_assert(R * THREADS == 512, "rows_per_workgroup assumes R * THREADS = 512");
-};
-// Rows per workgroup: the same for every layout and mode (R * THREADS = 512 lanes' rows).
-constexpr int rows_per_workgroup(int vbpr_log2) { return 512 >> vbpr_log2; }
+// R * THREADS / (N/16) rows per workgroup (64 rows = one Nemotron-H head at N = 128). Two rows per
+// lane in every layout and mode: four take 87 VGPRs in the reference layout (5 waves per SIMD; 42.2
+// against 41.4 us at batch 64), and in the compact layouts, where they once shared the
+// per-lane set-up over more rows (the head scalars, B and C come through LDS now), half as many
+// waves leave the chip idle at the middle batches: MX4 compact, batch 12 11.2 -> 9.1 us with two, 20
+// 14.4 -> 12.7; MX8 compact, batch 12 11.2 -> 9.1, 24 16.4 -> 14.8, 28 19.6 -> 16.6, 64 34.3 -> 34.0
+// us. The nibble layout keeps four rows per lane (in half as many threads, so the same workgroups)
+// for the largest grids, where they are still ahead: batch 48 (6144 workgroups) 24.8-25.0 against
+// 25.0, 64 31.7-32.0 against 32.1 us, deterministic 34.4 against 35.2 us.
+constexpr int ROWS_R = 2;
+constexpr int ROWS_THREADS = 256;
+constexpr int64_t WIDE_WORKGROUPS = 6144;
+constexpr int rows_per_workgroup(int vbpr_log2) { return ROWS_R * ROWS_THREADS >> vbpr_log2; }
 
 template <int FB, int RMODE, int BPR_LOG2, int LY>
 static void launch_rows_mode(const MxUpdateParams& p, dim3 grid, hipStream_t st) {
-  using G = RowsGeometry<LY, RMODE>;
-  hipLaunchKernelGGL((mx_update_rows_kernel<FB, RMODE, BPR_LOG2, G::R, G::THREADS, LY>), grid,
-                     dim3(G::THREADS), 0, st, p);
+  if constexpr (LY == LAYOUT_CM4 && RMODE != LQ_ROUND_SR_UNIFORM && RMODE != LQ_ROUND_SR_PHILOX) {
+    if ((int64_t)grid.x * grid.y * grid.z >= WIDE_WORKGROUPS) {
+      constexpr int R = 2 * ROWS_R, T = ROWS_THREADS / 2;
+      hipLaunchKernelGGL((mx_update_rows_kernel<FB, RMODE, BPR_LOG2, R, T, LY>), grid, dim3(T), 0, st, p);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((mx_update_rows_kernel<FB, RMODE, BPR_LOG2, ROWS_R, ROWS_THREADS, LY>), grid,
+                     dim3(ROWS_THREADS), 0, st, p);
 }
 
 template <int FB, int BPR_LOG2, int LY>
