@@ -228,6 +228,20 @@ int lq_int4_decode_attention_pack(const lq_tensor* q, const lq_tensor* k_new,
                                   void* stream);
 
 /*
+ * lq_int4_decode_attention_pack (with k_new and v_new) or lq_int4_decode_attention (both NULL)
+ * under a keep-mask, read as it is: keep [B, Lm] i64, required (any strides; keys whose value is 0
+ * and keys at or beyond Lm are masked). The cache bytes and the output equal those of the call with
+ * lq_keep_mask_bias's bias, without its launch and its array.
+ */
+int lq_int4_decode_attention_keep(const lq_tensor* q, const lq_tensor* k_new,
+                                  const lq_tensor* v_new, const lq_tensor* k_packed,
+                                  const lq_tensor* v_packed, const lq_tensor* k_scale,
+                                  const lq_tensor* v_scale, const lq_tensor* keep,
+                                  const lq_tensor* out, int64_t seq_len, int num_key_value_groups,
+                                  int group_size, void* workspace, size_t workspace_bytes,
+                                  void* stream);
+
+/*
  * lq_int4_decode_attention without a workspace: the same validation, kernels and results, with
  * the split-K partials in a static per-device buffer inside the library
  * (LQ_DECODE_ATTENTION_NOALLOC_SCRATCH_BYTES, 8 MiB on every GPU the library runs on, held until

@@ -69,6 +69,7 @@ EXPORTED_SYMBOLS = (
     "lq_int4_decode_attention_workspace",
     "lq_int4_decode_attention",
     "lq_int4_decode_attention_pack",
+    "lq_int4_decode_attention_keep",
     "lq_int4_decode_attention_noalloc",
     "lq_int4_prefill_attention",
     "lq_mx_encode",
@@ -128,6 +129,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.lq_int4_decode_attention_pack.argtypes = [_P] * 9 + [
         ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t,
         ctypes.c_void_p]
+    lib.lq_int4_decode_attention_keep.restype = ctypes.c_int
+    lib.lq_int4_decode_attention_keep.argtypes = [_P] * 9 + [
+        ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t,
+        ctypes.c_void_p]
     lib.lq_int4_decode_attention_noalloc.restype = ctypes.c_int
     lib.lq_int4_decode_attention_noalloc.argtypes = [_P] * 7 + [
         ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
@@ -176,7 +181,8 @@ def lib() -> ctypes.CDLL:
 # entry points that the host binding calls, in the order of its bind()
 _HOST_ENTRIES = (
     "lq_int4_pack_kv", "lq_int4_pack_kv_pair", "lq_int4_decode_attention_workspace",
-    "lq_int4_decode_attention", "lq_int4_decode_attention_pack", "lq_int4_prefill_attention",
+    "lq_int4_decode_attention", "lq_int4_decode_attention_pack",
+    "lq_int4_decode_attention_keep", "lq_int4_prefill_attention",
     "lq_mx_encode", "lq_mx_state_update", "lq_mx_state_update_device_step",
     "lq_selective_state_update", "lq_max_position", "lq_keep_mask_bias",
 )
@@ -477,6 +483,36 @@ def int4_decode_attention_pack(q: torch.Tensor, k_new: torch.Tensor, v_new: torc
         int(group_size), None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
         stream)
     check(rc, "lq_int4_decode_attention_pack")
+    return out
+
+
+def int4_decode_attention_keep(q: torch.Tensor, k_new: torch.Tensor | None,
+                               v_new: torch.Tensor | None, k_packed: torch.Tensor,
+                               v_packed: torch.Tensor, k_scale: torch.Tensor,
+                               v_scale: torch.Tensor, keep: torch.Tensor, out: torch.Tensor,
+                               seq_len: int, num_key_value_groups: int,
+                               group_size: int) -> torch.Tensor:
+    """int4_decode_attention_pack (without k_new and v_new: int4_decode_attention) under the int64
+    keep-mask [B, seq_len], which the kernel reads as it is."""
+    host = _host or host_binding()
+    if host:
+        rc = host.int4_decode_attention_keep(q, k_new, v_new, k_packed, v_packed, k_scale, v_scale,
+                                             keep, out, seq_len, num_key_value_groups, group_size,
+                                             _workspace.on_index)
+        if rc is not None:
+            check(rc, "lq_int4_decode_attention_keep")
+            return out
+    dev = _require_gpu(q, k_new, v_new, k_packed, v_packed, k_scale, v_scale, keep, out)
+    stream = _stream(dev)
+    need = int4_decode_attention_workspace(q.shape[0], q.shape[1], k_packed.shape[1],
+                                           q.shape[-1], seq_len, group_size)
+    ws = _workspace.get(dev, stream, need)
+    rc = lib().lq_int4_decode_attention_keep(
+        desc(q), desc(k_new), desc(v_new), desc(k_packed), desc(v_packed), desc(k_scale),
+        desc(v_scale), desc(keep), desc(out), int(seq_len), int(num_key_value_groups),
+        int(group_size), None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
+        stream)
+    check(rc, "lq_int4_decode_attention_keep")
     return out
 
 

@@ -22,6 +22,7 @@ struct Entries {
   decltype(&lq_int4_decode_attention_workspace) workspace;
   decltype(&lq_int4_decode_attention) attention;
   decltype(&lq_int4_decode_attention_pack) attention_pack;
+  decltype(&lq_int4_decode_attention_keep) attention_keep;
   decltype(&lq_int4_prefill_attention) prefill;
   decltype(&lq_mx_encode) encode;
   decltype(&lq_mx_state_update) update;
@@ -168,10 +169,13 @@ PyObject* py_pack_pair(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+enum AttentionCall { PLAIN, PACK_TOKEN, KEEP_MASK };
+
 // q, [k_new, v_new,] k_packed, v_packed, k_scale, v_scale, mask, out, seq_len, groups, group size,
 // and the workspace getter get(device index, stream handle, bytes) -> uint8 tensor
-template <bool PACK>
+template <AttentionCall CALL>
 PyObject* py_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  constexpr bool PACK = CALL != PLAIN;  // the call has the new token's rows (KEEP_MASK: or None)
   constexpr int NT = PACK ? 9 : 7;
   if (!has_args(n, NT + 4)) return nullptr;
   Tensors<NT> t;
@@ -207,8 +211,9 @@ PyObject* py_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Py_BEGIN_ALLOW_THREADS
   const lq_tensor* const* p = t.ptr;
   if constexpr (PACK) {
-    rc = entries.attention_pack(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], seq_len,
-                                nrep, g, ws, ws_bytes, stream);
+    const auto entry = CALL == KEEP_MASK ? entries.attention_keep : entries.attention_pack;
+    rc = entry(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], seq_len, nrep, g, ws,
+               ws_bytes, stream);
   } else {
     rc = entries.attention(p[0], p[1], p[2], p[3], p[4], p[5], p[6], seq_len, nrep, g, ws,
                            ws_bytes, stream);
@@ -333,8 +338,9 @@ PyObject* guarded(PyObject* self, PyObject* const* a, Py_ssize_t n) {
 PyMethodDef methods[] = {LQ_METHOD("bind", py_bind),
                          LQ_METHOD("int4_pack_kv", py_pack),
                          LQ_METHOD("int4_pack_kv_pair", py_pack_pair),
-                         LQ_METHOD("int4_decode_attention", py_attention<false>),
-                         LQ_METHOD("int4_decode_attention_pack", py_attention<true>),
+                         LQ_METHOD("int4_decode_attention", py_attention<PLAIN>),
+                         LQ_METHOD("int4_decode_attention_pack", py_attention<PACK_TOKEN>),
+                         LQ_METHOD("int4_decode_attention_keep", py_attention<KEEP_MASK>),
                          LQ_METHOD("int4_prefill_attention", py_prefill),
                          LQ_METHOD("mx_encode", py_encode),
                          LQ_METHOD("mx_state_update", py_update),

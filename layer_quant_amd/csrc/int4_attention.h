@@ -15,8 +15,11 @@ struct AttnParams {
   const float* ks;
   const float* vs;
   int64_t kss[4], vss[4];
-  const float* mask;  // NULL or [B, 1, 1, Lm] fp32 bias (batch and key strides used)
+  // NULL, an fp32 bias [B, 1, 1, Lm] (batch and key strides used), or (mask_keep) an int64 keep-mask
+  // [B, Lm] whose zeros count as -inf
+  const void* mask;
   int64_t mask_sb, mask_sk, mask_len;
+  bool mask_keep;
   View out;  // strides of (b, h, d)
   float* ws_m;
   float* ws_l;

@@ -79,7 +79,13 @@ __global__ __launch_bounds__(64) void attn_generic_kernel(AttnParams p) {
       }
       s = tot * p.scale_sm;
       if (p.mask != nullptr) {
-        s += (n < p.mask_len) ? p.mask[b * p.mask_sb + n * p.mask_sk] : -INFINITY;
+        float bias = -INFINITY;
+        if (n < p.mask_len) {
+          const int64_t i = b * p.mask_sb + n * p.mask_sk;
+          bias = !p.mask_keep ? ((const float*)p.mask)[i]
+                              : (((const int64_t*)p.mask)[i] != 0 ? 0.0f : -INFINITY);
+        }
+        s += bias;
       }
     }
     const float mt = group_max<64>(s);
@@ -388,7 +394,8 @@ static int decode_attention(const lq_tensor* q, const lq_tensor* k_packed,
                             const lq_tensor* v_packed, const lq_tensor* k_scale,
                             const lq_tensor* v_scale, const lq_tensor* mask, const lq_tensor* out,
                             int64_t seq_len, int num_key_value_groups, int group_size,
-                            PartialsBuffer buf, void* stream, NewToken tok = {nullptr, nullptr});
+                            PartialsBuffer buf, void* stream, NewToken tok = {nullptr, nullptr},
+                            bool keep = false);
 
 }  // namespace lq
 
@@ -435,6 +442,23 @@ extern "C" int lq_int4_decode_attention_pack(const lq_tensor* q, const lq_tensor
                           NewToken{k_new, v_new});
 }
 
+extern "C" int lq_int4_decode_attention_keep(const lq_tensor* q, const lq_tensor* k_new,
+                                             const lq_tensor* v_new, const lq_tensor* k_packed,
+                                             const lq_tensor* v_packed, const lq_tensor* k_scale,
+                                             const lq_tensor* v_scale, const lq_tensor* keep,
+                                             const lq_tensor* out, int64_t seq_len,
+                                             int num_key_value_groups, int group_size,
+                                             void* workspace, size_t workspace_bytes,
+                                             void* stream) {
+  if (keep == nullptr || (k_new == nullptr) != (v_new == nullptr)) {
+    return fail(LQ_ERR_INVALID_ARG, "keep is required, and k_new and v_new both or neither");
+  }
+  return decode_attention(q, k_packed, v_packed, k_scale, v_scale, keep, out, seq_len,
+                          num_key_value_groups, group_size,
+                          PartialsBuffer{workspace, workspace_bytes, false}, stream,
+                          NewToken{k_new, v_new}, true);
+}
+
 extern "C" int lq_int4_decode_attention_noalloc(const lq_tensor* q, const lq_tensor* k_packed,
                                                 const lq_tensor* v_packed,
                                                 const lq_tensor* k_scale,
@@ -453,7 +477,7 @@ static int decode_attention(const lq_tensor* q, const lq_tensor* k_packed,
                             const lq_tensor* v_packed, const lq_tensor* k_scale,
                             const lq_tensor* v_scale, const lq_tensor* mask, const lq_tensor* out,
                             int64_t seq_len, int num_key_value_groups, int group_size,
-                            PartialsBuffer buf, void* stream, NewToken tok) {
+                            PartialsBuffer buf, void* stream, NewToken tok, bool keep) {
   int rc;
   if (q == nullptr) return fail(LQ_ERR_INVALID_ARG, "q: descriptor is NULL");
   const int qdim = q->ndim;
@@ -508,7 +532,9 @@ static int decode_attention(const lq_tensor* q, const lq_tensor* k_packed,
                 (long long)seq_len, (long long)cap);
   }
   if (mask != nullptr) {
-    if ((rc = check_tensor(mask, "mask", 4, false, LQ_F32)) != LQ_OK) return rc;
+    rc = keep ? check_tensor(mask, "keep", 2, false, LQ_I64)
+              : check_tensor(mask, "mask", 4, false, LQ_F32);
+    if (rc != LQ_OK) return rc;
     if (mask->shape[0] != B) {
       return fail(LQ_ERR_INVALID_ARG, "mask batch %lld != %lld", (long long)mask->shape[0],
                   (long long)B);
@@ -543,10 +569,12 @@ static int decode_attention(const lq_tensor* q, const lq_tensor* k_packed,
     p.vss[i] = v_scale->stride[i];
   }
   if (mask != nullptr) {
-    p.mask = (const float*)mask->data;
+    const int last = mask->ndim - 1;
+    p.mask = mask->data;
+    p.mask_keep = keep;
     p.mask_sb = mask->stride[0];
-    p.mask_sk = mask->stride[3];
-    p.mask_len = mask->shape[3];
+    p.mask_sk = mask->stride[last];
+    p.mask_len = mask->shape[last];
   }
   p.out = make_view(out);
   p.B = (int)B;

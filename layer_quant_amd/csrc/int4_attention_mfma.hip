@@ -124,8 +124,14 @@ struct alignas(16) TileLds {
   u32x4_t v[2][64];
   float ks[TILE * 4];  // [key][group] (G <= 4)
   float vs[TILE * 4];
-  float mk[TILE];      // additive mask of the tile's keys (masked calls only)
+  // masked calls: the tile's additive mask (fp32), or its keep-mask (int64, two words per key)
+  uint32_t mk[2 * TILE];
 };
+
+// Mask of a call: none, additive fp32, or an int64 keep-mask (0 masks the key). The keep-mask is
+// the form that a serving loop has in hand: read here it costs 8 bytes per key where its bias costs
+// a launch and 4 (batch 8, 4001 keys: 16.9 us a step, 18.6 with the bias kernel before it).
+enum { MASK_NONE = 0, MASK_BIAS = 1, MASK_KEEP = 2 };
 
 typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
 
@@ -191,18 +197,18 @@ struct Rsrc {
   const float* ksb;
   const float* vsb;
   int kvo;  // this lane's source offset for the swizzled K slot
-  const float* mb;     // mask row of this batch (masked calls)
-  int msk_bytes;       // its key stride in bytes
+  const char* mb;      // mask row of this batch (masked calls)
+  int msk_bytes;       // its key stride in bytes (keep-mask: 8)
   int64_t mask_len;    // keys the mask covers
 };
 
 // Loads issued per tile (and counted by the waits): K 2, V 2, scales 2, and the mask row.
-template <bool MASK>
-constexpr int tile_loads() { return MASK ? 7 : 6; }
+template <int MASK>
+constexpr int tile_loads() { return MASK != MASK_NONE ? 7 : 6; }
 
 // Issue the loads of the tile at key tb into B (2 for K, 2 for V, one each for the K and V
 // scales on lanes below 8 G, and with MASK one for the tile's 32 mask values).
-template <int G, bool MASK>
+template <int G, int MASK>
 __device__ __forceinline__ void issue_tile(const Rsrc& R, int tb, int S, TileLds& B, int lane) {
   tb = __builtin_amdgcn_readfirstlane(tb);  // uniform by construction; descriptors in SGPRs
   const int rem = S - tb;  // > 0
@@ -231,12 +237,16 @@ __device__ __forceinline__ void issue_tile(const Rsrc& R, int tb, int S, TileLds
       load_to_lds_b32(rvs, &B.vs[0], 4 * lane);
     }
   }
-  if constexpr (MASK) {
+  if constexpr (MASK != MASK_NONE) {
     // keys at or past the mask's length read 0 here and are set to -inf by the score code
     const int64_t mrem = R.mask_len - tb;
-    const i32x4_t rm = make_desc(R.mb + (int64_t)tb * (R.msk_bytes >> 2),
+    const i32x4_t rm = make_desc(R.mb + (int64_t)tb * R.msk_bytes,
                                  mrem > 0 ? (int)mrem * R.msk_bytes : 0);
-    if (lane < TILE) load_to_lds_b32(rm, &B.mk[0], lane * R.msk_bytes);
+    if constexpr (MASK == MASK_KEEP) {
+      load_to_lds_b32(rm, &B.mk[0], 4 * lane);
+    } else {
+      if (lane < TILE) load_to_lds_b32(rm, &B.mk[0], lane * R.msk_bytes);
+    }
   }
 }
 
@@ -334,7 +344,7 @@ __device__ __forceinline__ void merge_unit(const AttnParams& p, int b, int kvh, 
   }
 }
 
-template <int NREP, int G, bool MASK>
+template <int NREP, int G, int MASK>
 __global__ __launch_bounds__(THREADS) void attn_fast_kernel(AttnParams p) {
   constexpr int LPT = tile_loads<MASK>();
   constexpr int NCOL = NREP * G;
@@ -382,8 +392,9 @@ __global__ __launch_bounds__(THREADS) void attn_fast_kernel(AttnParams p) {
   R.vsb = p.vs + b * p.vss[0] + kvh * p.vss[1];
   // K slot l of a half holds row l >> 2, unit (l & 3) ^ ((l >> 4) & 3)
   R.kvo = (lane >> 2) * 64 + 16 * ((lane & 3) ^ ((lane >> 4) & 3));
-  R.mb = MASK ? p.mask + b * p.mask_sb : nullptr;
-  R.msk_bytes = (int)(p.mask_sk * 4);
+  constexpr int MES = MASK == MASK_KEEP ? 8 : 4;  // bytes of a mask element
+  R.mb = MASK != MASK_NONE ? (const char*)p.mask + b * p.mask_sb * MES : nullptr;
+  R.msk_bytes = (int)(p.mask_sk * MES);
   R.mask_len = p.mask_len;
 
   // Fused pack (lq_int4_decode_attention_pack): the wave whose dealt tiles hold key S - 1 (its
@@ -590,10 +601,17 @@ __global__ __launch_bounds__(THREADS) void attn_fast_kernel(AttnParams p) {
       s[e] = column_sum<NREP>(sacc[e >> 2][e & 3], B.ks[key * G + colm]);
       vsc[e] = B.vs[key * G + colm];
     }
-    if constexpr (MASK) {  // additive mask in raw score units; keys past its length are -inf
+    if constexpr (MASK != MASK_NONE) {  // additive mask in raw score units; keys past its length are -inf
       float mv[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) mv[e] = B.mk[16 * (e >> 2) + 4 * (e & 3) + q4];
+      for (int e = 0; e < 8; ++e) {
+        const int key = 16 * (e >> 2) + 4 * (e & 3) + q4;
+        if constexpr (MASK == MASK_KEEP) {
+          mv[e] = (B.mk[2 * key] | B.mk[2 * key + 1]) != 0 ? 0.0f : -INFINITY;
+        } else {
+          mv[e] = __uint_as_float(B.mk[key]);
+        }
+      }
       if (tb + TILE <= p.mask_len) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) s[e] = fmaf(mv[e], inv_csm, s[e]);
@@ -804,10 +822,13 @@ bool fast_path_ok(const AttnParams& p) {
   if (((uintptr_t)p.ks & 3) != 0 || ((uintptr_t)p.vs & 3) != 0) return false;
   // buffer sizes of one (batch, KV head) block are 32-bit
   if (p.S * 64 >= ((int64_t)1 << 31)) return false;
-  // the mask row loads per lane with a 32-bit key stride and a 32-bit extent
+  // the mask row loads per lane with a 32-bit key stride and a 32-bit extent; a keep-mask's two
+  // words per key go to consecutive lanes, so its keys are dense
   if (p.mask != nullptr) {
+    const int64_t es = p.mask_keep ? 8 : 4;
     if (p.mask_sk <= 0 || ((uintptr_t)p.mask & 3) != 0) return false;
-    if (p.mask_len * p.mask_sk * 4 >= ((int64_t)1 << 31)) return false;
+    if (p.mask_keep && p.mask_sk != 1) return false;
+    if (p.mask_len * p.mask_sk * es >= ((int64_t)1 << 31)) return false;
   }
   return true;
 }
@@ -830,7 +851,7 @@ static FastResidency fast_residency() {
     }
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, reinterpret_cast<const void*>(&attn_fast_kernel<4, 4, false>), THREADS, 0) != hipSuccess ||
+            &per_cu, reinterpret_cast<const void*>(&attn_fast_kernel<4, 4, MASK_NONE>), THREADS, 0) != hipSuccess ||
         per_cu <= 0) {
       per_cu = 2;
     }
@@ -877,10 +898,12 @@ static void launch_one(AttnParams p, hipStream_t st) {
   p.grid3 = p.B <= 65535 && p.nsplit <= 65535;
   const dim3 grid = p.grid3 ? dim3((unsigned)p.Hkv, (unsigned)p.B, (unsigned)p.nsplit)
                             : dim3((unsigned)(p.B * p.Hkv), (unsigned)p.nsplit);
-  if (p.mask != nullptr) {
-    hipLaunchKernelGGL((attn_fast_kernel<NREP, G, true>), grid, dim3(THREADS), 0, st, p);
+  if (p.mask == nullptr) {
+    hipLaunchKernelGGL((attn_fast_kernel<NREP, G, MASK_NONE>), grid, dim3(THREADS), 0, st, p);
+  } else if (p.mask_keep) {
+    hipLaunchKernelGGL((attn_fast_kernel<NREP, G, MASK_KEEP>), grid, dim3(THREADS), 0, st, p);
   } else {
-    hipLaunchKernelGGL((attn_fast_kernel<NREP, G, false>), grid, dim3(THREADS), 0, st, p);
+    hipLaunchKernelGGL((attn_fast_kernel<NREP, G, MASK_BIAS>), grid, dim3(THREADS), 0, st, p);
   }
 }
 

@@ -159,6 +159,19 @@ def _decode_attention_mask(attention_mask: torch.Tensor | None, batch: int, seq_
         f"INT4 decode attention only supports 2D or 4D attention_mask, got {attention_mask.dim()}D")
 
 
+def _keep_rows(attention_mask: torch.Tensor | None, batch: int, seq_len: int,
+               device: torch.device) -> torch.Tensor | None:
+    """The last seq_len columns of an int64 keep-mask [batch, >= seq_len] on `device`, which the
+    decode kernel reads as they are: the attention of _decode_attention_mask's bias without its
+    launch. None for any other mask."""
+    if type(attention_mask) is not torch.Tensor or attention_mask.dim() != 2 \
+            or attention_mask.dtype != torch.int64 or attention_mask.device != device:
+        return None
+    cols = attention_mask[:, -seq_len:]
+    plain = cols.shape == (batch, seq_len) and cols.stride(1) == 1 and not cols.is_neg()
+    return cols if plain else None
+
+
 def _decode_attention(query_states: torch.Tensor, cache: Int4KVLayerCache, seq_len: int,
                       num_key_value_groups: int, group_size: int,
                       attention_mask: torch.Tensor | None = None) -> torch.Tensor:
@@ -169,6 +182,11 @@ def _decode_attention(query_states: torch.Tensor, cache: Int4KVLayerCache, seq_l
         raise ValueError(f"Fused INT4 decode attention expects q_len=1, got {q_len}")
     out = torch.empty((batch, n_heads, head_dim), device=query_states.device,
                       dtype=query_states.dtype)
+    keep = _keep_rows(attention_mask, batch, seq_len, query_states.device)
+    if keep is not None:
+        return _abi.int4_decode_attention_keep(query_states, None, None, cache.k_packed,
+                                               cache.v_packed, cache.k_scale, cache.v_scale, keep,
+                                               out, seq_len, num_key_value_groups, group_size)
     mask = _decode_attention_mask(attention_mask, batch, seq_len, query_states.device)
     _abi.int4_decode_attention(query_states, cache.k_packed, cache.v_packed, cache.k_scale,
                                cache.v_scale, mask, out, seq_len, num_key_value_groups,
@@ -188,6 +206,13 @@ def _pack_and_decode_attention(query_states: torch.Tensor, key_states: torch.Ten
         raise ValueError(f"Fused INT4 decode attention expects q_len=1, got {q_len}")
     out = torch.empty((batch, n_heads, head_dim), device=query_states.device,
                       dtype=query_states.dtype)
+    keep = _keep_rows(attention_mask, batch, seq_len, query_states.device)
+    if keep is not None:
+        _abi.int4_decode_attention_keep(query_states, key_states, value_states, cache.k_packed,
+                                        cache.v_packed, cache.k_scale, cache.v_scale, keep, out,
+                                        seq_len, num_key_value_groups, group_size)
+        cache.length = max(cache.length, seq_len)
+        return out
     try:
         mask = _decode_attention_mask(attention_mask, batch, seq_len, query_states.device)
     except ValueError:
