@@ -8,7 +8,8 @@
 //     (batch, query head, split), fp32 VALU throughout.
 // Scores follow the reference: s_n = (q . k_n) * log2(e)/sqrt(D) (+ mask_n), exp2-domain online
 // softmax; keys at or beyond the mask length get -inf. Splits write (m, l, acc[D]) partials into
-// the caller's workspace and attn_merge_kernel merges them; a single split writes out directly.
+// the caller's workspace and attn_merge_few_kernel merges them (attn_merge_kernel past 64 splits or
+// 256 dims); a single split writes out directly.
 // With LQ_DIAG_ATTN_FOLD_MERGE the MFMA kernel's last workgroup of each (batch, KV head) merges
 // them instead (counted by arrival counters at the start of the workspace): one launch, but at
 // batch 1 the kernel grows by more than the merge launch takes.

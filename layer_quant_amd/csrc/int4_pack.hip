@@ -143,7 +143,7 @@ __device__ __forceinline__ float group_absmax(const float (&v)[NV], bool& odd) {
 // in about one group of 15, so a product with v_rcp_f32 that sent lanes near a half-integer to the
 // division sent nearly every wave there (about 27 instructions per value; here about 8). K and V of
 // 16384 tokens, 8 heads, in the kernel trace: g = 32 26.3 -> 14.6 us (88 MB, 6.0 TB/s), g = 64
-// 28.5 -> 16.3, g = 128 (the row kernel) 30.4 -> 21.5 us.
+// 28.5 -> 16.3, g = 128 (then the row kernel) 30.4 -> 21.5 us.
 // The levels join as numbers: four give sum (k_i + 8) 16^i in [0, 65535], exact in fp32, in the low
 // 16 bits of that sum + 2^23 (three fmas and an add); the xor with 8 per nibble makes them two's
 // complement.
@@ -191,31 +191,32 @@ __device__ __forceinline__ uint32_t quantize8(const float (&v)[8], float& scale)
   return word[0];
 }
 
-// One lane per quantisation group of G values (16, 32 or 64) of a token row: G / 8 loads of 16
-// bytes (bf16 / fp16; twice that for fp32) issued together, the group's absmax within the lane,
-// and its G / 2 packed bytes written as 8- or 16-byte stores, its scale as one word: a wave reads
-// and writes whole consecutive rows. Rows contiguous (x stride 1 along head_dim, 16-byte aligned;
-// packed rows 16-byte aligned, or 8-byte for G = 16). Grid (lanes of one (batch, head) slice /
-// 256, B * H, tensors); head_dim / G = 2^lr_log2 lanes per token row.
-template <int G, int DT>
+// One lane per V values of a token row (16 or 32), L lanes per quantisation group of g = V * L: V / 8
+// loads of 16 bytes (bf16 / fp16; twice that for fp32) issued together, the group's absmax within the
+// lane and over its L lanes, V / 2 packed bytes written as an 8- or 16-byte store and the scale as
+// one word by the group's first lane: a wave reads and writes whole consecutive rows. Rows
+// contiguous (x stride 1 along head_dim, 16-byte aligned; packed rows 16-byte aligned, or 8-byte for
+// V = 16). Grid (lanes of one (batch, head) slice / 256, B * H, tensors); head_dim / V = 2^lr_log2
+// lanes per token row, a multiple of L.
+template <int V, int L, int DT>
 __global__ __launch_bounds__(256) void int4_pack_groups_kernel(PackPair pair, int lr_log2) {
   const PackParams& p = pair.pp[blockIdx.z];
   const int total = p.T << lr_log2;
   if (total == 0 || (int)blockIdx.y >= p.B * p.H) return;  // an empty or smaller tensor
   const int gid = (int)blockIdx.x * 256 + (int)threadIdx.x;
   const int g2 = min(gid, total - 1);
-  const int k = g2 & ((1 << lr_log2) - 1);  // group within the row
+  const int k = g2 & ((1 << lr_log2) - 1);  // lane within the row
   const int t = g2 >> lr_log2;
   const int b = (int)blockIdx.y / p.H;
   const int h = (int)blockIdx.y - b * p.H;
-  const int64_t xe = b * p.x.s[0] + h * p.x.s[1] + t * p.x.s[2] + G * k;
-  constexpr int NL = G / 8;
+  const int64_t xe = b * p.x.s[0] + h * p.x.s[1] + t * p.x.s[2] + V * k;
+  constexpr int NL = V / 8;
   // the token's row goes out with the values (loaded before the stores, it was one more round trip)
   const int64_t pos = p.positions != nullptr ? p.positions[t * p.pos_stride] : p.fixed_pos + t;
   Raw8<DT> raw[NL];
 #pragma unroll
   for (int i = 0; i < NL; ++i) raw[i] = load8<DT>(p.x.data, xe + 8 * i);
-  float v[G];
+  float v[V];
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
     float w[8];
@@ -224,21 +225,25 @@ __global__ __launch_bounds__(256) void int4_pack_groups_kernel(PackPair pair, in
     for (int u = 0; u < 8; ++u) v[8 * i + u] = w[u];
   }
   bool odd;
-  const float scale = fmaxf(group_absmax<G>(v, odd) / 7.0f, 1.0e-8f);
-  uint32_t words[G / 8];
-  pack_levels<G>(v, scale, odd, words);
+  float amax = group_absmax<V>(v, odd);
+  // every lane of the wave is here; a group's lanes are all in or all past the slice's end
+#pragma unroll
+  for (int o = L >> 1; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+  const float scale = fmaxf(amax / 7.0f, 1.0e-8f);
+  uint32_t words[V / 8];
+  pack_levels<V>(v, scale, odd, words);
   if (gid >= total || pos < 0 || pos >= p.cap) return;
-  uint8_t* dst = p.packed + b * p.ps[0] + h * p.ps[1] + pos * p.ps[2] + (G / 2) * k;
-  if constexpr (G == 16) {
+  uint8_t* dst = p.packed + b * p.ps[0] + h * p.ps[1] + pos * p.ps[2] + (V / 2) * k;
+  if constexpr (V == 16) {
     *(uint2*)dst = make_uint2(words[0], words[1]);
   } else {
 #pragma unroll
-    for (int w = 0; w < G / 32; ++w) {
+    for (int w = 0; w < V / 32; ++w) {
       *(uint4*)(dst + 16 * w) = make_uint4(words[4 * w], words[4 * w + 1], words[4 * w + 2],
                                            words[4 * w + 3]);
     }
   }
-  p.scale[b * p.ss[0] + h * p.ss[1] + pos * p.ss[2] + k * p.ss[3]] = scale;
+  if (k % L == 0) p.scale[b * p.ss[0] + h * p.ss[1] + pos * p.ss[2] + (k / L) * p.ss[3]] = scale;
 }
 
 // One lane per 8 values of a token row (dims 8j .. 8j + 7 -> packed bytes 4j .. 4j + 3) in each
@@ -382,11 +387,17 @@ int make_pack_params(const lq_tensor* x, const lq_tensor* packed, const lq_tenso
 
 int64_t pack_bytes(const PackParams& p) { return (int64_t)p.B * p.H * p.T * (p.D / 2); }
 
-// int4_pack_groups_kernel's layout: g of 16, 32 or 64 and head_dim / g a power of two, the row
+// Values per lane of int4_pack_groups_kernel, larger groups on several lanes. K and V of 16384
+// tokens, 8 heads: g = 128 14.6 us on four lanes of 32 (16.4 on two of 64; 21.6 in the row kernel's 16
+// lanes of 8), g = 64 15.0 on two of 32 against 16.5 on one of 64 (300 tokens: 4.0 against 4.8):
+// twice the waves, and half the stride between the lanes' 16-byte loads.
+constexpr int GROUP_LANE_VALUES = 32;
+
+// int4_pack_groups_kernel's layout: g of 16, 32, 64 or 128 and head_dim / g a power of two, the row
 // kernel's layout otherwise, and packed rows aligned to the lane's stores (16 bytes; 8 for g = 16).
 bool rows_layout_ok(const PackPair& pair, int n, int group_size);
 bool groups_layout_ok(const PackPair& pair, int n, int group_size) {
-  if (group_size != 16 && group_size != 32 && group_size != 64) return false;
+  if (group_size != 16 && group_size != 32 && group_size != 64 && group_size != 128) return false;
   if (!rows_layout_ok(pair, n, group_size)) return false;
   const int al = group_size == 16 ? 8 : 16;
   for (int i = 0; i < n; ++i) {
@@ -447,28 +458,30 @@ int launch_pack(const PackPair& pair, int n, int group_size, hipStream_t s, cons
   // for a few tokens per slice (a decode token) most of their lanes would idle, and the
   // one-lane-per-byte kernel's flat grid fills the waves instead.
   const bool many_rows = slice_rows * (pair.pp[0].D / 8) >= 256;
+  const int values = std::min(group_size, GROUP_LANE_VALUES);
   if (many_rows && groups_layout_ok(pair, n, group_size) &&
-      slice_rows * (pair.pp[0].D / group_size) < ((int64_t)1 << 31) - 256 && slices <= 65535) {
-    const int lr_log2 = __builtin_ctz((unsigned)(pair.pp[0].D / group_size));
+      slice_rows * (pair.pp[0].D / values) < ((int64_t)1 << 31) - 256 && slices <= 65535) {
+    const int lr_log2 = __builtin_ctz((unsigned)(pair.pp[0].D / values));
     const int64_t lanes = slice_rows << lr_log2;
     const dim3 grid((unsigned)((lanes + 255) / 256), (unsigned)slices, (unsigned)n);
     const int dt = pair.pp[0].x.dtype;
     auto go = [&](auto gv) {
-      constexpr int GV = decltype(gv)::value;
+      constexpr int G = decltype(gv)::value, V = std::min(G, GROUP_LANE_VALUES), L = G / V;
       if (dt == LQ_BF16) {
-        hipLaunchKernelGGL((int4_pack_groups_kernel<GV, LQ_BF16>), grid, dim3(256), 0, s, pair,
+        hipLaunchKernelGGL((int4_pack_groups_kernel<V, L, LQ_BF16>), grid, dim3(256), 0, s, pair,
                            lr_log2);
       } else if (dt == LQ_F16) {
-        hipLaunchKernelGGL((int4_pack_groups_kernel<GV, LQ_F16>), grid, dim3(256), 0, s, pair,
+        hipLaunchKernelGGL((int4_pack_groups_kernel<V, L, LQ_F16>), grid, dim3(256), 0, s, pair,
                            lr_log2);
       } else {
-        hipLaunchKernelGGL((int4_pack_groups_kernel<GV, LQ_F32>), grid, dim3(256), 0, s, pair,
+        hipLaunchKernelGGL((int4_pack_groups_kernel<V, L, LQ_F32>), grid, dim3(256), 0, s, pair,
                            lr_log2);
       }
     };
     if (group_size == 16) go(std::integral_constant<int, 16>{});
     else if (group_size == 32) go(std::integral_constant<int, 32>{});
-    else go(std::integral_constant<int, 64>{});
+    else if (group_size == 64) go(std::integral_constant<int, 64>{});
+    else go(std::integral_constant<int, 128>{});
     return check_launch(what);
   }
   constexpr int RROWS = 4;  // rows per lane

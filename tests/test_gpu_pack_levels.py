@@ -40,3 +40,33 @@ def test_prompt_levels_equal_token_levels(gpu, dtype, g):
         _abi.int4_pack_kv(x[:, :, i:i + 1], *token, torch.tensor([i], device=gpu), g)
     assert torch.equal(prompt[0], token[0])
     assert torch.equal(prompt[1], token[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("d,g", [(64, 64), (128, 64), (128, 128), (256, 128), (512, 64)])
+@pytest.mark.parametrize("t", [32, 33, 71, 130])
+def test_groups_over_several_lanes(gpu, dtype, d, g, t):
+    """Groups that span lanes: odd token counts end inside a workgroup, a group's values in one lane
+    only (its neighbours zero, NaN or infinite), positions in any order and outside the cache."""
+    b, h, cap = 2, 2, t + 3
+    gen = torch.Generator().manual_seed(d + g + t)
+    x = torch.stack([_values(max(t, 48), d, dtype, gen)[:t] if d > 70 else
+                     torch.randn(t, d, generator=gen).to(dtype) for _ in range(b * h)])
+    x[:, 5] = 0
+    x[:, 5, d - 1] = 3  # the scale comes from the group's last lane
+    x[:, 6, : d // 2] = float("inf")
+    x = x.view(b, h, t, d).to(gpu)
+    pos = torch.randperm(cap, generator=gen)[:t]
+    pos[1], pos[2] = -1, cap
+    pos = pos.to(gpu)
+
+    def cache():
+        return (torch.full((b, h, cap, d // 2), 9, dtype=torch.uint8, device=gpu),
+                torch.full((b, h, cap, d // g), -1.0, device=gpu))
+
+    prompt, token = cache(), cache()
+    _abi.int4_pack_kv(x, *prompt, pos, g)
+    for i in range(t):  # one token per call: the one-lane-per-byte kernel
+        _abi.int4_pack_kv(x[:, :, i:i + 1], *token, pos[i:i + 1], g)
+    assert torch.equal(prompt[0], token[0])
+    assert torch.equal(prompt[1], token[1])
