@@ -6,20 +6,45 @@
 namespace lq {
 
 constexpr int MAX_THREADS = 1024;
+constexpr int MAX_LOADS = 8;  // loads of a thread that are in flight together
 
-// One workgroup: each thread's loads go out eight at a time, then a shuffle reduction per wave and
-// one over the waves. The result is stored with system scope to pinned host memory, so no copy
-// follows. 16384 positions: 4.4 us, one 2.4 us (torch's reduction 7.2 and 2.6 us, then a copy). The
-// call that packs 16384 tokens, which waits for it: 34.4 -> 23.7 us, most of it from not waiting for
-// the pack.
+// The largest of m and what load(0 .. n - 1) brings in (one or two positions each), MAX_LOADS per thread
+// at a time; past the end the last one again, so that every batch is one round trip.
+template <typename T, typename Load>
+__device__ __forceinline__ int64_t thread_max(int64_t m, int64_t n, Load load) {
+  for (int64_t i0 = threadIdx.x; i0 - threadIdx.x < n; i0 += (int64_t)MAX_LOADS * blockDim.x) {
+    T v[MAX_LOADS];
+#pragma unroll
+    for (int u = 0; u < MAX_LOADS; ++u) v[u] = load(min(i0 + (int64_t)u * blockDim.x, n - 1));
+#pragma unroll
+    for (int u = 0; u < MAX_LOADS; ++u) {
+      if constexpr (sizeof(T) == 16) {
+        m = max(m, max((int64_t)v[u].x, (int64_t)v[u].y));
+      } else {
+        m = max(m, (int64_t)v[u]);
+      }
+    }
+  }
+  return m;
+}
+
+// One workgroup: each thread's loads (16 bytes where the positions are dense and aligned) go out eight
+// at a time, then a shuffle reduction per wave and one over the waves. The result is stored with system scope to pinned host memory, so no copy
+// follows. 16384 positions: 3.3 us, 65536 6.0, one 2.4 (8-byte loads under an unrolled loop, whose
+// remainder went one at a time, 4.4 and 9.6 us; torch's reduction 7.2 us for 16384, then a copy). The call
+// that packs 16384 tokens, which waits for it: 34.4 -> 22.8 us, most of it from not waiting for the
+// pack.
 __global__ __launch_bounds__(MAX_THREADS) void max_position_kernel(const int64_t* pos,
                                                                    int64_t stride, int64_t n,
                                                                    int64_t* host_slot) {
   __shared__ int64_t part[MAX_THREADS / 64];
   const int tid = threadIdx.x;
-  int64_t m = pos[0];
-#pragma unroll 8
-  for (int64_t i = tid; i < n; i += blockDim.x) m = max(m, pos[i * stride]);
+  int64_t m = pos[(n - 1) * stride];  // the last of an odd count has no pair
+  if (stride == 1 && ((uintptr_t)pos & 15) == 0) {
+    m = thread_max<longlong2>(m, n >> 1, [&](int64_t i) { return ((const longlong2*)pos)[i]; });
+  } else {
+    m = thread_max<int64_t>(m, n, [&](int64_t i) { return pos[i * stride]; });
+  }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) m = max(m, (int64_t)__shfl_xor((long long)m, o, 64));
   if ((tid & 63) == 0) part[tid >> 6] = m;

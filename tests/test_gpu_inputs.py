@@ -36,6 +36,19 @@ def test_max_position(gpu, n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("offset", [0, 1])  # 16-byte aligned or not
+@pytest.mark.parametrize("n", [1, 2, 3, 511, 512, 513, 2047, 4095, 8193, 16383, 16384, 16385, 65535])
+def test_max_position_anywhere(gpu, n, offset):
+    buf = torch.full((n + 2,), 1 << 50, dtype=torch.int64, device=gpu)  # neighbours are larger
+    pos = buf[offset:offset + n]
+    pos.copy_(torch.arange(n, device=gpu) - n)
+    for at in {0, n // 2, n - 2, n - 1} - {-1}:
+        pos[at] += 1 << 41
+        assert _abi.start_max_position(pos).wait() == (1 << 41) + at - n
+        pos[at] -= 1 << 41
+
+
+@pytest.mark.gpu
 def test_max_position_follows_its_stream(gpu):
     """The value is the one the positions hold when the stream gets there, on any stream."""
     side = torch.cuda.Stream()
