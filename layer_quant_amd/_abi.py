@@ -324,10 +324,12 @@ def int4_pack_kv_pair(k: torch.Tensor, v: torch.Tensor, k_packed: torch.Tensor,
 
 
 class _PendingMax:
-    """One thread's pinned slot and event on one device. wait() ends the use that start() began;
-    the owner calls it before start() is called again, also when the work in between raises."""
+    """A pinned slot and an event on one device. wait() ends the use that start() began and gives the
+    slot back to the thread's free ones; the owner calls it once, also when the work in between
+    raises."""
 
-    def __init__(self):
+    def __init__(self, free: list):
+        self._free = free
         self._pinned = torch.zeros(1, dtype=torch.int64, pin_memory=True)
         self.address = self._pinned.data_ptr()
         self._value = ctypes.c_int64.from_address(self.address)
@@ -338,15 +340,20 @@ class _PendingMax:
 
     def wait(self) -> int:
         self._event.synchronize()
-        return self._value.value
+        value = self._value.value
+        self._free.append(self)
+        return value
 
 
-class _PendingMaxima(threading.local):
+class _FreeSlots(threading.local):
+    """The slots a thread has in hand per device: as many as it once had pending together, which is
+    one, or more where a module that runs between start and wait makes such a call itself."""
+
     def __init__(self):
-        self.by_device: dict[int, _PendingMax] = {}
+        self.by_device: dict[int, list[_PendingMax]] = {}
 
 
-_pending_maxima = _PendingMaxima()
+_free_slots = _FreeSlots()
 # above this, torch's reduction over many workgroups is the faster one
 MAX_POSITIONS = 1 << 16
 
@@ -357,19 +364,20 @@ def start_max_position(positions) -> _PendingMax | None:
     is not a plain 1-D int64 tensor on a GPU, or the stream is being captured: the caller then
     uses positions.max().item()."""
     if type(positions) is not torch.Tensor or positions.dtype != torch.int64 \
-            or positions.dim() != 1 or not positions.is_cuda \
+            or positions.dim() != 1 or not positions.is_cuda or positions.is_neg() \
             or not 1 <= positions.numel() <= MAX_POSITIONS:
         return None
     host = _host or host_binding()
     if not host or torch.cuda.is_current_stream_capturing():
         return None
     device = positions.get_device()
-    pending = _pending_maxima.by_device.get(device)
-    if pending is None:
-        pending = _pending_maxima.by_device[device] = _PendingMax()
+    free = _free_slots.by_device.setdefault(device, [])
+    pending = free.pop() if free else _PendingMax(free)
     rc = host.max_position(positions, pending.address)
-    if rc is None:
-        return None
+    if rc != LQ_OK:  # nothing was launched
+        free.append(pending)
+        if rc is None:
+            return None
     check(rc, "lq_max_position")
     pending.record(device)
     return pending

@@ -29,11 +29,11 @@ __device__ __forceinline__ int64_t thread_max(int64_t m, int64_t n, Load load) {
 }
 
 // One workgroup: each thread's loads (16 bytes where the positions are dense and aligned) go out eight
-// at a time, then a shuffle reduction per wave and one over the waves. The result is stored with system scope to pinned host memory, so no copy
-// follows. 16384 positions: 3.3 us, 65536 6.0, one 2.4 (8-byte loads under an unrolled loop, whose
-// remainder went one at a time, 4.4 and 9.6 us; torch's reduction 7.2 us for 16384, then a copy). The call
-// that packs 16384 tokens, which waits for it: 34.4 -> 22.8 us, most of it from not waiting for the
-// pack.
+// at a time, then a shuffle reduction per wave and one over the waves. The result is stored with system
+// scope to pinned host memory, so no copy follows. 16384 positions: 3.3 us, 65536 6.0, one 2.4 (8-byte
+// loads under an unrolled loop, whose remainder went one at a time, 4.4 and 9.6 us; torch's reduction
+// 7.2 us for 16384, then a copy). The call that packs 16384 tokens, which waits for it: 34.4 -> 22.8
+// us, most of it from not waiting for the pack.
 __global__ __launch_bounds__(MAX_THREADS) void max_position_kernel(const int64_t* pos,
                                                                    int64_t stride, int64_t n,
                                                                    int64_t* host_slot) {

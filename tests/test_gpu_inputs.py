@@ -68,6 +68,23 @@ def test_max_position_follows_its_stream(gpu):
 
 
 @pytest.mark.gpu
+def test_max_positions_pending_together(gpu):
+    """A second read started before the first one's wait (a projection that is itself such a call)
+    keeps its own value; the slots are taken again afterwards."""
+    pos = [torch.full((n,), n, dtype=torch.int64, device=gpu) for n in (3, 50, 700)]
+    for _ in range(3):
+        started = [_abi.start_max_position(p) for p in pos]
+        assert [s.wait() for s in started] == [3, 50, 700]
+    free = _abi._free_slots.by_device[gpu.index or 0]
+    held = len(free)
+    assert held >= 3
+    for _ in range(3):
+        assert _abi.start_max_position(pos[0]).wait() == 3
+    assert len(free) == held
+    assert _abi.start_max_position(torch._neg_view(pos[0])) is None
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bool, torch.uint8, torch.int8, torch.int16, torch.int32,
                                    torch.int64, torch.float16, torch.bfloat16, torch.float32,
                                    torch.float64])
