@@ -250,16 +250,17 @@ __global__ __launch_bounds__(1024) void attn_merge_few_kernel(const float* __res
     m[i] = ws_m[base + min(g + i * groups, ns - 1)];
     l[i] = ws_l[base + min(g + i * groups, ns - 1)];
   }
-  float M = m[0];  // (a repeated last split changes no maximum; its weight below is 0)
+  float M = m[0];  // (a repeated last split changes no maximum; below it is left out)
 #pragma unroll
   for (int i = 1; i < NS; ++i) M = fmaxf(M, m[i]);
   float L = 0.0f, acc = 0.0f;
 #pragma unroll
   for (int i = 0; i < NS; ++i) {
-    const bool in = g + i * groups < ns && m[i] != -INFINITY;
-    const float w = in ? __builtin_amdgcn_exp2f(m[i] - M) : 0.0f;
-    L += w * l[i];
-    acc += w * part[i];
+    if (g + i * groups < ns) {  // (uniform; an infinite partial of a repeated split times 0 is NaN)
+      const float w = m[i] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[i] - M);
+      L += w * l[i];
+      acc += w * part[i];
+    }
   }
   if (groups > 1) {
     s_acc[threadIdx.x] = acc;
