@@ -226,7 +226,8 @@ __global__ __launch_bounds__(MERGE_THREADS) void attn_merge_kernel(AttnParams p)
 // threads holds dim d of one (batch, query head) over the splits g, g + groups, ... Its partials and
 // the splits' m and l (the same for every lane of a wave: scalar loads) all go out at once, and every
 // lane makes the weights itself: one memory round trip and no reduction across lanes; more than one
-// group joins through LDS. With two block reductions before the weights (attn_merge_kernel) the launch
+// group joins through LDS. The weights are exp2f's, as in attn_merge_kernel: the bare instruction
+// makes those below 2^-126 zero, and a split of large values behind such a weight was lost. With two block reductions before the weights (attn_merge_kernel) the launch
 // took 3.9 us in the kernel trace at 8 splits, batch 1, and 4.4 at 32; here 2.9 and 3.9 us. (All of
 // 32 splits in one thread: 8.8 us.)
 template <int NS>
@@ -257,7 +258,7 @@ __global__ __launch_bounds__(1024) void attn_merge_few_kernel(const float* __res
 #pragma unroll
   for (int i = 0; i < NS; ++i) {
     if (g + i * groups < ns) {  // (uniform; an infinite partial of a repeated split times 0 is NaN)
-      const float w = m[i] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[i] - M);
+      const float w = m[i] == -INFINITY ? 0.0f : exp2f(m[i] - M);
       L += w * l[i];
       acc += w * part[i];
     }
@@ -274,7 +275,7 @@ __global__ __launch_bounds__(1024) void attn_merge_few_kernel(const float* __res
     for (int i = 1; i < groups; ++i) Mt = fmaxf(Mt, s_m[i]);
     L = acc = 0.0f;
     for (int i = 0; i < groups; ++i) {
-      const float w = s_m[i] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(s_m[i] - Mt);
+      const float w = s_m[i] == -INFINITY ? 0.0f : exp2f(s_m[i] - Mt);
       L += w * s_l[i];
       acc += w * s_acc[i * width + t];
     }

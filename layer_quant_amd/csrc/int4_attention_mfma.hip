@@ -731,7 +731,7 @@ __global__ __launch_bounds__(THREADS) void attn_fast_kernel(AttnParams p) {
   }
   __syncthreads();
 
-  // merge the 4 waves
+  // merge the 4 waves (exp2f: weights below 2^-126 count where a wave's values are large)
   for (int idx = tid; idx < NREP * FAST_D; idx += THREADS) {
     const int h = idx / FAST_D;
     const int d = idx - h * FAST_D;
@@ -743,7 +743,7 @@ __global__ __launch_bounds__(THREADS) void attn_fast_kernel(AttnParams p) {
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
       const float mw = o_wave(w)[NREP * FAST_D + h];
-      const float wt = (mw == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(mw - M);
+      const float wt = (mw == -INFINITY) ? 0.0f : exp2f(mw - M);
       L += wt * o_wave(w)[NREP * FAST_D + NREP + h];
       a += wt * o_wave(w)[h * FAST_D + d];
     }

@@ -1,5 +1,5 @@
-"""The decode attention's split merge at the end of fp32's range: infinite partials beside finite
-ones."""
+"""The decode attention's merges at the ends of fp32's range: infinite partials beside finite ones,
+and weights below the smallest normal number."""
 import pytest
 import torch
 
@@ -37,3 +37,20 @@ def test_infinite_partial_stays_infinite(gpu, diag, splits, where):
     out, ref = _run(gpu, torch.randn(1, 4, 1, d, generator=gen), k, v, 32)
     assert torch.isposinf(out[..., :32]).all()
     assert_close_rel(out[..., 32:], ref[..., 32:], what=f"splits={splits}")
+
+
+@pytest.mark.parametrize("fast,s,cold", [(False, 64 * n - 5, 64) for n in (2, 9, 33, 65)]
+                         + [(True, 128, 32), (True, 128 * 2, 128), (True, 128 * 20 - 7, 128)])
+def test_subnormal_weight_of_large_values(gpu, diag, fast, s, cold):
+    """The first `cold` keys score 127.5 below the others (in powers of two), and their values are
+    2^126 times larger, so that their subnormal weight still makes a quarter of the result or more. They are
+    one split's keys, or (fast, 128 keys) one wave's tile of 32."""
+    diag.set("LQ_ATTN_REQUIRE_FAST" if fast else "LQ_ATTN_FORCE_GENERIC")
+    gen = torch.Generator().manual_seed(s)
+    q = torch.full((1, 4, 1, 128), 7.8125, dtype=torch.bfloat16)  # q . k = 1000 for k = 1
+    k, v = torch.ones(1, 2, s, 128), torch.randn(1, 2, s, 128, generator=gen)
+    k[:, :, :cold] = 0.0
+    v[:, :, :cold] = v[:, :, :cold].abs() * 2.0 ** 118
+    v[:, :, cold:] *= 2.0 ** -8
+    out, ref = _run(gpu, q, k, v, 32)
+    assert_close_rel(out, ref, what=f"fast={fast} S={s}")
