@@ -844,18 +844,13 @@ static FastResidency fast_residency() {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return FastResidency{256, 2};
   if (cached[dev].cus == 0) {
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        cus <= 0) {
-      cus = 256;
-    }
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
             &per_cu, reinterpret_cast<const void*>(&attn_fast_kernel<4, 4, MASK_NONE>), THREADS, 0) != hipSuccess ||
         per_cu <= 0) {
       per_cu = 2;
     }
-    cached[dev] = FastResidency{cus, per_cu};
+    cached[dev] = FastResidency{device_cus(), per_cu};
   }
   return cached[dev];
 }

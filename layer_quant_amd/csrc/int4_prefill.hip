@@ -238,8 +238,8 @@ __device__ __forceinline__ uint32_t out_bits(float v, int dtype) {
 
 // KS key groups of NW waves: group kg takes the tiles kg, kg + KS, ... of the workgroup's keys, each
 // group staging its own; with KS = 2 wave w of both groups holds the same query rows, and at the end
-// each hands the other one of its two column tiles and finishes the other (launch_mfma's rule says
-// when that pays). QV and OV: the query and output rows take 16-byte accesses.
+// each hands the other one of its two column tiles and finishes the other (two_key_groups says when
+// that pays). QV and OV: the query and output rows take 16-byte accesses.
 template <int G, int KS, bool QV, bool OV>
 __global__ __launch_bounds__(64 * NW * KS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void prefill_mfma_kernel(PrefillParams p) {
@@ -385,7 +385,7 @@ void prefill_mfma_kernel(PrefillParams p) {
     for (int i = 0; i < 8; ++i) o[qt][i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
   }
 
-  // (a key group past the last tile stages zeros from beyond key L and skips them: tb >= wend)
+  // (a key group past the last tile stages the last one again and has to skip it: tb >= wend)
   for (int st = 0; st < nsteps; st += KS) {
     const int nb = (st / KS) & 1;
     __syncthreads();  // this step's tiles are staged; the other buffers are free
@@ -719,13 +719,25 @@ bool rows_aligned(const View& v) {
 // 16384 4143 -> 3970 us; batch 2, L = 777 63.7 -> 56.0 us. (More than 65535 position blocks do not
 // fit grid.y and keep the position blocks in grid.x.)
 //
-// Two key groups (KS = 2) while every workgroup finds a slot of two per CU anyway (256 CUs): the
-// time is then that of the longest chain of tile steps, which two groups halve. L = 777, batch 2
-// 43.0 -> 37.4 us; batch 1, L = 500 32.2 -> 26.5, 1024 57.0 -> 44.3, 1500 72.0 -> 52.2, 2048 (512
-// workgroups) 112.6 -> 91.5 us. With more workgroups the independent four-wave ones are faster
-// (their waves are in different phases of a step): batch 4, L = 600 (608 workgroups) 42.4 against
-// 56.2 us, batch 1, L = 3000 165 against 194, 8192 1023 against 1165 us.
-constexpr int64_t KS2_WORKGROUPS = 512;
+// Two key groups (KS = 2) halve the longest chain of tile steps, but one workgroup of eight waves
+// fills a CU (182-224 VGPRs, two waves per SIMD), so that a grid of more workgroups than CUs runs in
+// two generations, and the second one's prologue and epilogue cost about 9 us (one tile, group 32: 256
+// workgroups 12.3 us, 320 21.9). The line is the measured crossover on 256 CUs, for groups of 32 to 128
+// and 1 to 8 heads per KV head: a call goes by its workgroups and tiles whatever its batch and heads
+// (KS = 1 -> 2, us, group 64):
+//   up to a workgroup per CU, from 3 tiles: batch 1, L = 1024 48.5 -> 39.9; batch 8, L = 128 14.1 ->
+//     13.5 (2 tiles 11.7 -> 12.0, 1 tile 10.7 -> 11.6)
+//   up to two per CU, where the chain is long beside the grid: batch 1, L = 2048 91.9 -> 77.5; batch
+//     2, L = 777 41.5 -> 37.0, 1024 52.4 -> 48.7; batch 3, L = 400 26.0 -> 23.8, 640 37.1 -> 37.5;
+//     not batch 4, L = 300 22.2 -> 22.4, 512 32.2 -> 33.9; batch 8, L = 256 21.8 -> 26.2; batch 16,
+//     L = 80 14.0 -> 20.6; batch 64, L = 16 12.0 -> 18.9
+//   above that not: batch 4, L = 600 (608 workgroups) 42.4 -> 56.2, batch 1, L = 3000 165 -> 194,
+//     8192 1023 -> 1165 (group 32)
+bool two_key_groups(int64_t workgroups, int64_t tiles) {
+  const int64_t cus = device_cus();
+  if (workgroups <= cus) return tiles >= 3;
+  return workgroups <= 2 * cus && workgroups <= 24 * tiles;
+}
 
 template <int G, int KS>
 void launch_mfma_ks(const PrefillParams& p, dim3 grid, hipStream_t st) {
@@ -751,7 +763,7 @@ void launch_mfma(PrefillParams p, hipStream_t st) {
   p.unit_fast = nwg <= 65535;
   const dim3 grid = p.unit_fast ? dim3((unsigned)units, (unsigned)nwg)
                                 : dim3((unsigned)nwg, (unsigned)units);
-  if (nwg * units <= KS2_WORKGROUPS) {
+  if (two_key_groups(nwg * units, npb)) {
     launch_mfma_ks<G, 2>(p, grid, st);
   } else {
     launch_mfma_ks<G, 1>(p, grid, st);

@@ -17,6 +17,9 @@ void set_error(const char* fmt, ...) __attribute__((format(printf, 1, 2)));
 int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 int check_launch(const char* what);
 
+// CUs of the current device (256, an MI355X's, where the runtime does not say).
+int device_cus();
+
 inline int dtype_size(int dtype) {
   switch (dtype) {
     case LQ_U8:

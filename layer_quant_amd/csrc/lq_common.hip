@@ -41,6 +41,21 @@ int check_launch(const char* what) {
   return LQ_OK;
 }
 
+int device_cus() {
+  static std::atomic<int> cached[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int cus = cached[dev].load(std::memory_order_relaxed);
+  if (cus == 0) {
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        cus <= 0) {
+      cus = 256;
+    }
+    cached[dev].store(cus, std::memory_order_relaxed);
+  }
+  return cus;
+}
+
 int check_tensor(const lq_tensor* t, const char* name, int ndim, bool float_dtype,
                  int exact_dtype) {
   if (t == nullptr) return fail(LQ_ERR_INVALID_ARG, "%s: descriptor is NULL", name);
