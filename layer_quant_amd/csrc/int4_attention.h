@@ -40,6 +40,19 @@ struct AttnParams {
   int grid3;     // MFMA path: grid (KV heads, batch, splits) instead of (units, splits)
 };
 
+// Weight 2^(m - M) of a partial with maximum m under the merged maximum M, 0 for one without a key
+// (m = -inf). By exp2f: the bare instruction makes results below 2^-126 zero, and a partial of large
+// values behind such a weight would be lost. Its six instructions are the reason why the merges make
+// each weight in one lane and hand it out.
+__device__ __forceinline__ float partial_weight(float m, float M) {
+  return m == -INFINITY ? 0.0f : exp2f(m - M);
+}
+
+// A lane's value in every lane (lane uniform).
+__device__ __forceinline__ float from_lane(float v, int lane) {
+  return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane));
+}
+
 struct SplitPlan {
   int nsplit;
   int64_t chunk;

@@ -21,6 +21,8 @@
 #include <atomic>
 #include <mutex>
 
+#include <type_traits>
+
 #include "int4_attention.h"
 #include "int4_quant.h"
 
@@ -222,20 +224,34 @@ __global__ __launch_bounds__(MERGE_THREADS) void attn_merge_kernel(AttnParams p)
   }
 }
 
+// v combined over the 16 lanes of a row, in every lane of it.
+template <class F>
+__device__ __forceinline__ float row_reduce(float v, F op) {
+  auto ror = [&](auto n) {
+    const int r = __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + n.value, 0xf, 0xf, false);
+    v = op(v, __int_as_float(r));
+  };
+  ror(std::integral_constant<int, 8>{});
+  ror(std::integral_constant<int, 4>{});
+  ror(std::integral_constant<int, 2>{});
+  ror(std::integral_constant<int, 1>{});
+  return v;
+}
+
 // The same for at most NS * groups splits and D <= 256: thread d of each group of blockDim.x / groups
-// threads holds dim d of one (batch, query head) over the splits g, g + groups, ... Its partials and
-// the splits' m and l (the same for every lane of a wave: scalar loads) all go out at once, and every
-// lane makes the weights itself: one memory round trip and no reduction across lanes; more than one
-// group joins through LDS. The weights are exp2f's, as in attn_merge_kernel: the bare instruction
-// makes those below 2^-126 zero, and a split of large values behind such a weight was lost. With two block reductions before the weights (attn_merge_kernel) the launch
-// took 3.9 us in the kernel trace at 8 splits, batch 1, and 4.4 at 32; here 2.9 and 3.9 us. (All of
-// 32 splits in one thread: 8.8 us.)
+// threads holds dim d of one (batch, query head) over the splits g, g + groups, ..., and lane i of
+// each row of 16 lanes the i-th one's m and l. All go out at once: one memory round trip, no
+// reduction past a row; more than one group joins through LDS. With two block reductions before the
+// weights (attn_merge_kernel) the launch took 3.9 us in the kernel trace at 8 splits, batch 1, and
+// 4.4 at 32; here 2.7 and 3.8 us (every lane making every weight by exp2f 3.4 at 8 splits). (All of 32
+// splits in one thread: 8.8 us.)
 template <int NS>
 __global__ __launch_bounds__(1024) void attn_merge_few_kernel(const float* __restrict__ ws_m,
                                                               const float* __restrict__ ws_l,
                                                               const float* __restrict__ ws_acc,
                                                               View out, int Hq, int D, int ns,
                                                               int groups) {
+  static_assert(NS <= 16, "a row of lanes holds a group's splits");
   __shared__ float s_acc[1024], s_m[MERGE_GROUPS], s_l[MERGE_GROUPS];
   const int bh = blockIdx.x;
   const int64_t base = (int64_t)bh * ns;
@@ -243,26 +259,23 @@ __global__ __launch_bounds__(1024) void attn_merge_few_kernel(const float* __res
   const int g = __builtin_amdgcn_readfirstlane((int)threadIdx.x / width);
   const int t = (int)threadIdx.x - g * width;
   const int d = min(t, D - 1);
-  float part[NS], m[NS], l[NS];
+  float part[NS];
 #pragma unroll
   for (int i = 0; i < NS; ++i) part[i] = ws_acc[(base + min(g + i * groups, ns - 1)) * D + d];
+  const int mine = g + ((int)threadIdx.x & 15) * groups;  // this lane's split
+  const float m0 = ws_m[base + min(mine, ns - 1)], l0 = ws_l[base + min(mine, ns - 1)];
+  const float m = mine < ns ? m0 : -INFINITY;
+  const float M = row_reduce(m, [](float a, float b) { return fmaxf(a, b); });
+  const float w = partial_weight(m, M);
+  float L = row_reduce(mine < ns ? w * l0 : 0.0f, [](float a, float b) { return a + b; });
+  if (g + (NS - 1) * groups >= ns) {
+    // the splits past the end, loaded as the last one again, whose partial may be infinite
 #pragma unroll
-  for (int i = 0; i < NS; ++i) {
-    m[i] = ws_m[base + min(g + i * groups, ns - 1)];
-    l[i] = ws_l[base + min(g + i * groups, ns - 1)];
+    for (int i = 1; i < NS; ++i) part[i] = g + i * groups < ns ? part[i] : 0.0f;
   }
-  float M = m[0];  // (a repeated last split changes no maximum; below it is left out)
+  float acc = 0.0f;
 #pragma unroll
-  for (int i = 1; i < NS; ++i) M = fmaxf(M, m[i]);
-  float L = 0.0f, acc = 0.0f;
-#pragma unroll
-  for (int i = 0; i < NS; ++i) {
-    if (g + i * groups < ns) {  // (uniform; an infinite partial of a repeated split times 0 is NaN)
-      const float w = m[i] == -INFINITY ? 0.0f : exp2f(m[i] - M);
-      L += w * l[i];
-      acc += w * part[i];
-    }
-  }
+  for (int i = 0; i < NS; ++i) acc += from_lane(w, i) * part[i];
   if (groups > 1) {
     s_acc[threadIdx.x] = acc;
     if (t == 0) {
@@ -275,9 +288,9 @@ __global__ __launch_bounds__(1024) void attn_merge_few_kernel(const float* __res
     for (int i = 1; i < groups; ++i) Mt = fmaxf(Mt, s_m[i]);
     L = acc = 0.0f;
     for (int i = 0; i < groups; ++i) {
-      const float w = s_m[i] == -INFINITY ? 0.0f : exp2f(s_m[i] - Mt);
-      L += w * s_l[i];
-      acc += w * s_acc[i * width + t];
+      const float wg = partial_weight(s_m[i], Mt);
+      L += wg * s_l[i];
+      acc += wg * s_acc[i * width + t];
     }
   }
   if (t >= D) return;

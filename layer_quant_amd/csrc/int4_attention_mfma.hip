@@ -731,22 +731,26 @@ __global__ __launch_bounds__(THREADS) void attn_fast_kernel(AttnParams p) {
   }
   __syncthreads();
 
-  // merge the 4 waves (exp2f: weights below 2^-126 count where a wave's values are large)
-  for (int idx = tid; idx < NREP * FAST_D; idx += THREADS) {
-    const int h = idx / FAST_D;
-    const int d = idx - h * FAST_D;
-    float M = -INFINITY;
+  // merge the 4 waves: lane l makes the weights of head l mod NREP
+  float hm[WAVES], wt[WAVES];
+  float hM = -INFINITY, hL = 0.0f;
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) M = fmaxf(M, o_wave(w)[NREP * FAST_D + h]);
-    float L = 0.0f;
+  for (int w = 0; w < WAVES; ++w) {
+    hm[w] = o_wave(w)[NREP * FAST_D + lane % NREP];
+    hM = fmaxf(hM, hm[w]);
+  }
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    wt[w] = partial_weight(hm[w], hM);
+    hL += wt[w] * o_wave(w)[NREP * FAST_D + NREP + lane % NREP];
+  }
+  for (int idx = tid; idx < NREP * FAST_D; idx += THREADS) {
+    const int h = __builtin_amdgcn_readfirstlane(idx / FAST_D);  // one head per wave and pass
+    const int d = idx - h * FAST_D;
+    const float M = from_lane(hM, h), L = from_lane(hL, h);
     float a = 0.0f;
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-      const float mw = o_wave(w)[NREP * FAST_D + h];
-      const float wt = (mw == -INFINITY) ? 0.0f : exp2f(mw - M);
-      L += wt * o_wave(w)[NREP * FAST_D + NREP + h];
-      a += wt * o_wave(w)[h * FAST_D + d];
-    }
+    for (int w = 0; w < WAVES; ++w) a += from_lane(wt[w], h) * o_wave(w)[h * FAST_D + d];
     const int qh = kvh * NREP + h;
     if (p.nsplit == 1) {
       store_float(p.out.data, p.out.dtype, b * p.out.s[0] + qh * p.out.s[1] + d * p.out.s[2],
