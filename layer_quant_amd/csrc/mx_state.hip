@@ -1309,14 +1309,17 @@ static void dispatch_encode(const MxCodecParams& p, int rmode, bool vec, dim3 gr
 
 // Rows kernel geometry: R rows per lane, THREADS threads, one (batch, head) slice of up to
 // R * THREADS / (N/16) rows per workgroup (64 rows = one Nemotron-H head at N = 128). Two rows per
-// lane in every layout and mode: four take 87 VGPRs in the reference layout (5 waves per SIMD; 42.2
-// against 41.4 us at batch 64), and in the compact layouts, where they once shared the
-// per-lane set-up over more rows (the head scalars, B and C come through LDS now), half as many
-// waves leave the chip idle at the middle batches: MX4 compact, batch 12 11.2 -> 9.1 us with two, 20
+// lane: four take 87 VGPRs in the reference layout (5 waves per SIMD; 42.2 against 41.4 us at batch
+// 64), and in the compact layouts, where they once shared the per-lane set-up over more rows (the
+// head scalars, B and C come through LDS now), half as many waves leave the chip idle at the middle batches: MX4 compact, batch 12 11.2 -> 9.1 us with two, 20
 // 14.4 -> 12.7; MX8 compact, batch 12 11.2 -> 9.1, 24 16.4 -> 14.8, 28 19.6 -> 16.6, 64 34.3 -> 34.0
-// us. The nibble layout keeps four rows per lane (in half as many threads, so the same workgroups)
-// for the largest grids, where they are still ahead: batch 48 (6144 workgroups) 24.8-25.0 against
-// 25.0, 64 31.7-32.0 against 32.1 us, deterministic 34.4 against 35.2 us.
+// us. The nibble layout at N = 128 keeps four rows per lane (in half as many threads, so the same
+// workgroups) for the largest grids, where they are still ahead, by 1-3 % (two -> four, us, medians of
+// four alternated runs of 128 heads x 64 rows, stochastic / deterministic): batch 48 (6144 workgroups)
+// 30.8 -> 30.2 / 29.4 -> 29.0, 64 36.2 -> 35.7 / 34.9 -> 34.3, 96 52.4 -> 50.9 / 50.5 -> 50.2, 128
+// 67.2 -> 65.5 / 66.1 -> 64.9 (24 heads, batch 256 26.2 -> 26.8 / 26.3 -> 26.8, inside the runs'
+// spread). Not at the other widths: N = 64, batch 64 29.1 -> 29.3 / 25.6 -> 25.4; N = 256, batch 64
+// 66.8 -> 69.0 / 66.9 -> 66.4.
 constexpr int ROWS_R = 2;
 constexpr int ROWS_THREADS = 256;
 constexpr int64_t WIDE_WORKGROUPS = 6144;
@@ -1324,7 +1327,8 @@ constexpr int rows_per_workgroup(int vbpr_log2) { return ROWS_R * ROWS_THREADS >
 
 template <int FB, int RMODE, int BPR_LOG2, int LY>
 static void launch_rows_mode(const MxUpdateParams& p, dim3 grid, hipStream_t st) {
-  if constexpr (LY == LAYOUT_CM4 && RMODE != LQ_ROUND_SR_UNIFORM && RMODE != LQ_ROUND_SR_PHILOX) {
+  if constexpr (LY == LAYOUT_CM4 && BPR_LOG2 == 3 && RMODE != LQ_ROUND_SR_UNIFORM &&
+                RMODE != LQ_ROUND_SR_PHILOX) {
     if ((int64_t)grid.x * grid.y * grid.z >= WIDE_WORKGROUPS) {
       constexpr int R = 2 * ROWS_R, T = ROWS_THREADS / 2;
       hipLaunchKernelGGL((mx_update_rows_kernel<FB, RMODE, BPR_LOG2, R, T, LY>), grid, dim3(T), 0, st, p);
