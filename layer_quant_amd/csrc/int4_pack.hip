@@ -3,13 +3,19 @@
 // Replaces _pack_int4_kv_kernel (reference hybrid_quant/int4_8b_attention.py:32-111). Per group
 // of g values along head_dim: absmax -> scale = max(absmax / 7, 1e-8) -> q = rint(x / scale)
 // (IEEE division, round half to even) -> clamp [-8, 7] -> two's-complement nibbles, even d in the
-// low nibble. int4_pack_lanes_kernel gives one lane to each output byte (dims 2j, 2j+1), so a
-// group is g/2 adjacent lanes and its absmax a shuffle reduction; int4_pack_kernel (one thread
-// per group) covers group sizes whose g/2 is not a power of two up to 64. int4_pack_rows_kernel
-// takes the common layout (contiguous rows, 16-byte aligned, g a multiple of 8): one lane per 8
-// values of each of 4 rows (16- or 32-byte loads issued together, 4-byte stores), g/8 lanes per
-// group, and the division by the scale done as a corrected product with its reciprocal, which gives
-// the same levels (pack_levels).
+// low nibble. Four kernels (launch_pack chooses):
+//   int4_pack_groups_kernel  prompts with contiguous 16-byte aligned rows, g = 16, 32, 64 or 128:
+//                            16 or 32 values per lane, 8- and 16-byte stores
+//   int4_pack_rows_kernel    prompts with such rows of any g that is 8 times a power of two (8, 256 and
+//                            512 in practice), or whose packed rows are only 4-byte aligned: one
+//                            lane per 8 values of each of 4 rows (16- or 32-byte loads issued
+//                            together, 4-byte stores), g/8 lanes per group
+//   int4_pack_lanes_kernel   decode tokens and every other view, g/2 a power of two up to 64: one
+//                            lane per output byte (dims 2j, 2j+1), so a group is g/2 adjacent lanes
+//                            and its absmax a shuffle reduction
+//   int4_pack_kernel         the rest: one thread per group
+// The first two divide by the scale as a corrected product with its reciprocal, which gives the same
+// levels (pack_levels).
 // All kernels take up to two tensors (blockIdx.y picks one): lq_int4_pack_kv_pair packs a layer's
 // K and V in one launch.
 #include <algorithm>

@@ -70,3 +70,24 @@ def test_groups_over_several_lanes(gpu, dtype, d, g, t):
         _abi.int4_pack_kv(x[:, :, i:i + 1], *token, pos[i:i + 1], g)
     assert torch.equal(prompt[0], token[0])
     assert torch.equal(prompt[1], token[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("g", [16, 32, 64, 128])
+def test_packed_rows_aligned_to_words_only(gpu, dtype, g):
+    """Packed rows 68 bytes apart from an offset of 4: the kernel with 4-byte stores at the group sizes
+    that aligned caches take to the one with wide stores. Nothing is written between the rows."""
+    b, h, t, d = 1, 2, 77, 128
+    gen = torch.Generator().manual_seed(g)
+    x = torch.stack([_values(t, d, dtype, gen) for _ in range(b * h)]).view(b, h, t, d).to(gpu)
+    pos = torch.arange(t, device=gpu)
+    buf = torch.full((4 + b * h * t * 68,), 9, dtype=torch.uint8, device=gpu)
+    rows = buf[4:].view(b, h, t, 68)
+    token = torch.zeros(b, h, t, d // 2, dtype=torch.uint8, device=gpu)
+    scale, token_scale = (torch.zeros(b, h, t, d // g, device=gpu) for _ in range(2))
+    _abi.int4_pack_kv(x, rows[..., :d // 2], scale, pos, g)
+    for i in range(t):  # one token per call: the one-lane-per-byte kernel
+        _abi.int4_pack_kv(x[:, :, i:i + 1], token, token_scale, pos[i:i + 1], g)
+    assert torch.equal(rows[..., :d // 2], token)
+    assert torch.equal(scale, token_scale)
+    assert (buf[:4] == 9).all() and (rows[..., d // 2:] == 9).all()
