@@ -706,6 +706,15 @@ __global__ __launch_bounds__(THREADS) void attn_fast_kernel(AttnParams p) {
     process(i + 2, tiles2[wave]);
   }
 
+  // From here on the arguments are read again from the kernel's argument segment (p, the only one, is
+  // at its start). Read with the others, before the loop, they were held over it in scalar registers,
+  // which run out: the loop then reloads spilled ones (3 more instructions per tile, batch 61, ctx
+  // 16000, g 64 186.7 -> 190.4 us; read again 187.6).
+  typedef const __attribute__((address_space(4))) void* kernarg_t;
+  kernarg_t kernarg = (kernarg_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(kernarg));
+  const AttnParams& pe = *(const AttnParams*)kernarg;
+
   // per-wave partial -> LDS (in the wave's first tile buffer, whose last reads are complete)
   // wave w's partial: o [NREP][FAST_D], then m [NREP] and l [NREP]
   auto o_wave = [&](int w) -> float* {
@@ -752,27 +761,27 @@ __global__ __launch_bounds__(THREADS) void attn_fast_kernel(AttnParams p) {
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) a += from_lane(wt[w], h) * o_wave(w)[h * FAST_D + d];
     const int qh = kvh * NREP + h;
-    if (p.nsplit == 1) {
-      store_float(p.out.data, p.out.dtype, b * p.out.s[0] + qh * p.out.s[1] + d * p.out.s[2],
+    if (pe.nsplit == 1) {
+      store_float(pe.out.data, pe.out.dtype, b * pe.out.s[0] + qh * pe.out.s[1] + d * pe.out.s[2],
                   a / L);
     } else {
-      const int64_t slot = ((int64_t)b * p.Hq + qh) * p.nsplit + split;
-      if (p.fold) {
-        coherent_store(&p.ws_acc[slot * FAST_D + d], a);
+      const int64_t slot = ((int64_t)b * pe.Hq + qh) * pe.nsplit + split;
+      if (pe.fold) {
+        coherent_store(&pe.ws_acc[slot * FAST_D + d], a);
         if (d == 0) {
-          coherent_store(&p.ws_m[slot], M);
-          coherent_store(&p.ws_l[slot], L);
+          coherent_store(&pe.ws_m[slot], M);
+          coherent_store(&pe.ws_l[slot], L);
         }
       } else {
-        p.ws_acc[slot * FAST_D + d] = a;
+        pe.ws_acc[slot * FAST_D + d] = a;
         if (d == 0) {
-          p.ws_m[slot] = M;
-          p.ws_l[slot] = L;
+          pe.ws_m[slot] = M;
+          pe.ws_l[slot] = L;
         }
       }
     }
   }
-  if (p.nsplit > 1 && p.fold) {
+  if (pe.nsplit > 1 && pe.fold) {
     // Folded split-K merge: the last of the unit's nsplit workgroups to arrive merges all of
     // them and puts the unit's counter back to 0, so a call leaves every counter as it found it.
     // No workgroup waits for another. The partials go through device-coherent accesses (written
@@ -786,13 +795,13 @@ __global__ __launch_bounds__(THREADS) void attn_fast_kernel(AttnParams p) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (tid == 0) {
-      s_last = __hip_atomic_fetch_add(&p.ws_cnt[unit], 1u, __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(p.nsplit - 1);
+      s_last = __hip_atomic_fetch_add(&pe.ws_cnt[unit], 1u, __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(pe.nsplit - 1);
     }
     __syncthreads();
     if (!s_last) return;
-    merge_unit<NREP>(p, b, kvh, s_w, s_wl, s_L);
-    if (tid == 0) __hip_atomic_store(&p.ws_cnt[unit], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    merge_unit<NREP>(pe, b, kvh, s_w, s_wl, s_L);
+    if (tid == 0) __hip_atomic_store(&pe.ws_cnt[unit], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
