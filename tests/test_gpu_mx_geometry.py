@@ -1,5 +1,5 @@
 """The MX row kernel's two lane geometries: on both sides of the grid size where the nibble layout
-goes from two to four rows per lane, the compact update equals the reference layout's bit for bit."""
+goes from two to four rows per lane (d_state 128; the other widths stay at two), the compact update equals the reference layout's bit for bit."""
 import pytest
 import torch
 
